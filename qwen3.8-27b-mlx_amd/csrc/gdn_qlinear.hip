@@ -75,6 +75,10 @@ struct QParams {
   // per group, so a workgroup's m tiles of one group are one run
   float* xsum;
   int mtiles;
+  // MFMA path: xfrag in 32-row fragments instead (qgemm_big_kernel): (L, mtiles / 2, K / 64, 4)
+  // blocks of 64 lanes x 8 bf16; lane 32 h + mm of block s of group g holds row 32 mb + mm,
+  // values k = 64 g + 32 h + 8 s + (0, 4, 1, 5, 2, 6, 3, 7)
+  int frag32;
   int mgroups;  // MFMA path: groups of MT m-tiles (the grid is layers x tiles x mgroups)
   int remap;    // MFMA path: XCD-aware workgroup order (see qgemm_kernel)
 };
@@ -319,8 +323,13 @@ __global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p, int layers) 
   u32x4 q;
 #pragma unroll
   for (int e = 0; e < 4; ++e) q[e] = pack_bf2(v[e], v[e + 4]);
-  const int f = 2 * (c / 2) + (j & 1), ln = 16 * (2 * (c & 1) + j / 2) + (mrow & 15);
-  *reinterpret_cast<u32x4*>(blk + ((size_t)f * 64 + ln) * 8) = q;
+  if (p.frag32) {
+    uint16_t* b32 = p.xfrag + ((size_t)layer * (p.mtiles / 2) + mrow / 32) * nch * 1024;
+    *reinterpret_cast<u32x4*>(b32 + ((size_t)(4 * (c / 2) + j) * 64 + 32 * (c & 1) + (mrow & 31)) * 8) = q;
+  } else {
+    const int f = 2 * (c / 2) + (j & 1), ln = 16 * (2 * (c & 1) + j / 2) + (mrow & 15);
+    *reinterpret_cast<u32x4*>(blk + ((size_t)f * 64 + ln) * 8) = q;
+  }
   // the group's sum x: the 64 values of (row, group c / 2) are the 8 values of each of 8
   // consecutive threads (pieces c, c + 1 of a group are adjacent: nch is even), added in
   // a fixed order (each thread's 8 in sequence, then a butterfly over the 8 threads)
@@ -412,7 +421,9 @@ __device__ __forceinline__ RowPtrs row_ptrs(const QParams& p, int layer, int row
 // below), and the workgroup's scale and bias pairs are staged in LDS once at the start
 // (they would otherwise be two more loads per row tile and group at the same depth).
 constexpr int kRing = 2;  // groups in flight per wave (G / 4 is a multiple of it)
-template <int MT, int NT>
+// F32: the operand is in qgemm_big_kernel's 32-row fragments (its leftover rows): this lane's
+// values are block 2 (g4 % 2) + s of group g there, lane 32 (g4 / 2) + 16 (mt % 2) + nn.
+template <int MT, int NT, bool F32>
 __global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
   constexpr int kRows = 16 * NT;
   constexpr int kMaxG = 8192 / 64;
@@ -463,7 +474,8 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
     const RowPtrs rl = row_ptrs(p, layer, lrow < p.R ? lrow : p.R - 1);
     wr[nt] = (g_u32x2*)(rl.w) + (lane & 3);  // + 4 g: words 8 g + 2 c, +1
   }
-  const bf8* xa = reinterpret_cast<const bf8*>(p.xfrag + ((size_t)layer * p.mtiles + mt0) * nch * 512) + lane;
+  const bf8* xa = reinterpret_cast<const bf8*>(p.xfrag + ((size_t)layer * p.mtiles + mt0) * nch * 512) +
+                  (F32 ? 128 * (g4 & 1) + 32 * (g4 >> 1) + nn : lane);
   const NibbleConsts nk = nibble_consts();
 
   // A ring of kRing slots, one group each (operand fragments and nibble words): slot j
@@ -479,7 +491,9 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) sl.a[mt][s] = xa[((size_t)mt * nch + 2 * g + s) * 64];
+      for (int s = 0; s < 2; ++s)
+        sl.a[mt][s] = F32 ? xa[((size_t)(mt / 2) * nch * 2 + 4 * g + s) * 64 + 16 * (mt & 1)]
+                          : xa[((size_t)mt * nch + 2 * g + s) * 64];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) sl.w[nt] = wr[nt][4 * g];
   };
@@ -609,10 +623,41 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 }
 __device__ __forceinline__ void dma16(const void* src, uint32_t lds) {
   uint32_t m0_saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_nop 0\n\ts_mov_b32 m0, %0"
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
                : "=&s"(m0_saved)
                : "v"(src), "s"(lds)
                : "memory");
+}
+// four consecutive 1 KB blocks from a wave-uniform address (the instruction offset moves both
+// addresses); voff = 16 x lane
+__device__ __forceinline__ void dma16x4(const void* src, uint32_t voff, uint32_t lds) {
+  uint32_t m0_saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+               "global_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\t"
+               "global_load_lds_dwordx4 %1, %2 offset:2048\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072\n\t"
+               "s_mov_b32 m0, %0"
+               : "=&s"(m0_saved)
+               : "v"(voff), "s"(src), "s"(lds)
+               : "memory");
+}
+// two consecutive blocks from one uniform address, a lane's source offsets v0 and v1
+__device__ __forceinline__ void dma16x2(const void* src, uint32_t v0, uint32_t v1, uint32_t lds) {
+  uint32_t m0_saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\t"
+               "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(m0_saved)
+               : "v"(v0), "v"(v1), "s"(src), "s"(lds)
+               : "memory", "scc");
+}
+// one block where `skip` (wave-uniform) is 0; the branch is inside the asm, so that the
+// compiler's basic block -- and the order of the products and sums in it -- stays whole
+__device__ __forceinline__ void dma16_unless(int skip, const void* src, uint32_t voff, uint32_t lds) {
+  uint32_t m0_saved;
+  asm volatile("s_cmp_lg_u32 %4, 0\n\ts_cbranch_scc1 1f\n\t"
+               "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0\n1:"
+               : "=&s"(m0_saved)
+               : "v"(voff), "s"(src), "s"(lds), "s"(skip)
+               : "memory", "scc");
 }
 
 template <int MT>
@@ -835,6 +880,335 @@ __global__ __launch_bounds__(kThreads) void qgemm_ns_kernel(QParams p) {
     }
 }
 
+// MFMA path for many operand rows: an LDS-tiled product on v_mfma_f32_32x32x16_bf16.
+// Workgroup = 4 waves as WN x WK over a tile of 32 MTW operand rows x 64 WN weight rows of one
+// matrix; the WK wave sets take every WK-th group of K and add their sums in LDS at the end.
+// Two workgroups share a CU (80 KB of LDS each), so that one's barriers fall into the other's
+// products. A step is WK groups: its operand blocks (16 KB) and nibble words (8 KB) pass
+// through a ring of kBigSlots LDS slots filled by direct-to-LDS loads ahead of their use; each
+// wave's scale words come 8 groups at a time into its own pair of buffers. Per group and
+// 32 x 32 tile: four products into acc = sum x (16 + q), then y += s acc (16 FMAs a lane
+// beside 128 cycles of MFMA); the bias term is made before the loop on MFMA, as
+// qgemm_ns_kernel does after its. Nibble q is the bf16 16 + q here (q in the mantissa's upper
+// four bits: one shift more per word than 128 + q): the terms of the offset are summed apart
+// from the products that cancel them, so their size is what the fp32 sums round at, and with
+// 128 the outputs lay further from the exact product than qgemm_kernel's, which cancels them
+// group by group (with 16 they lie as near or nearer).
+typedef float f16v __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f16v mfma32(bf8 a, bf8 b, f16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// Nibble word (values k .. k + 7) as a B fragment: bf16 16 + v, pairs (i, i + 4).
+__device__ __forceinline__ NibbleConsts nibble16_consts() {
+  NibbleConsts k;
+  k.mask = 0x00780078u;
+  k.bias = 0x41804180u;
+  asm volatile("" : "+v"(k.mask), "+v"(k.bias));
+  return k;
+}
+__device__ __forceinline__ bf8 nibbles16_bf16(uint32_t wd, NibbleConsts k) {
+  u32x4 r;
+  r[0] = and_or(wd << 3, k.mask, k.bias);
+#pragma unroll
+  for (int q = 1; q < 4; ++q) r[q] = and_or(wd >> (4 * q - 3), k.mask, k.bias);
+  return __builtin_bit_cast(bf8, r);
+}
+constexpr int kBigSlots = 3;
+template <int WN, int WK, int MTW>
+struct BigCfg {
+  static constexpr int NTW = 2;                    // 32-row weight tiles of a wave
+  static constexpr int kRows = 64 * WN;            // weight rows of the tile
+  static constexpr int kABytes = MTW * WK * 4096;  // operand bytes of a step
+  static constexpr int kWBytes = WN * WK * 2048;   // nibble bytes of a step
+  static constexpr int kSlot = kABytes + kWBytes;
+  static constexpr int kPerStep = 6;               // loads of a wave and step: 4 + 2
+  static constexpr int kSbStride = 8 / WK;         // steps an 8-group block of scale words lasts
+  static constexpr size_t kLds = kBigSlots * kSlot + 4 * 2 * 1024;
+  static_assert(WN * WK == 4 && MTW * WK == 4, "4 waves share each step's loads evenly");
+};
+
+template <int WN, int WK, int MTW>
+__global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
+  using C = BigCfg<WN, WK, MTW>;
+  constexpr int NTW = C::NTW;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[C::kLds];
+  unsigned char* const ring = smem;
+  uint16_t* const sbl_all = reinterpret_cast<uint16_t*>(smem + kBigSlots * C::kSlot);  // [wave][2][64 rows][8 groups]
+  // Workgroups are dispatched to the XCDs round robin: each XCD takes a contiguous range of
+  // tile ids, in which panels of 8 weight tiles run weight tile fastest, so the tiles one XCD
+  // runs at once share their weight and operand slices through its L2.
+  int bid = blockIdx.x;
+  if (p.remap) bid = (bid & 7) * (int)(gridDim.x >> 3) + (bid >> 3);
+  const int per_layer = p.tiles * p.mgroups;
+  const int layer = bid / per_layer;
+  int rem = bid % per_layer;
+  const int panel = rem / (8 * p.mgroups);
+  const int width = min(8, p.tiles - 8 * panel);
+  rem -= panel * 8 * p.mgroups;
+  const int tile = 8 * panel + rem % width, mg = rem / width;
+
+  // the tile's matrix (row0 counts whole tiles here) and its base addresses, wave-uniform
+  const uint32_t* wseg = p.w[0];
+  const uint16_t *sseg = p.s[0], *bseg = p.b[0];
+  uint16_t* yseg = p.y[0];
+  int nseg = p.n[0], t0 = 0;
+#pragma unroll
+  for (int q = 1; q < GDN_QLINEAR_MAX_SEGS; ++q) {
+    if (q < p.nseg && tile >= p.row0[q]) {
+      wseg = p.w[q];
+      sseg = p.s[q];
+      bseg = p.b[q];
+      yseg = p.y[q];
+      nseg = p.n[q];
+      t0 = p.row0[q];
+    }
+  }
+  const int lane = threadIdx.x & 63, h = lane >> 5, nn = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave % WK, wn = wave / WK;
+  const int G = p.K / 64, nsteps = G / WK, nblk = G / 8;
+  const int mblk = p.mtiles / 2;  // the operand's 32-row blocks
+  const int mb0 = mg * MTW;
+  const int nbase = (tile - t0) * C::kRows + 64 * wn;  // this wave's first row of the matrix
+  const size_t wrow = (size_t)p.K / 2;                 // bytes of a weight row
+  const char* const wb = reinterpret_cast<const char*>(wseg) + (size_t)layer * nseg * wrow;
+  const char* const sb = reinterpret_cast<const char*>(sseg) + (size_t)layer * nseg * (2 * G);
+  const char* const bb_ = reinterpret_cast<const char*>(bseg) + (size_t)layer * nseg * (2 * G);
+
+  // this wave's loads of a step: the four blocks of one (group, operand block) and the nibble
+  // words of its own 64 rows and group in two loads of 32 rows, a lane pair the 32 bytes of a
+  // row (the halves of rows 4..7 of every 8 swapped: eight lanes of a read then hit distinct
+  // banks). Offsets of lanes in a matrix: 32 bits (the host checks it).
+  const int a_kg = wave / MTW, a_mb = wave % MTW;
+  const char* const a_src = reinterpret_cast<const char*>(p.xfrag) +
+                            (((size_t)layer * mblk + min(mb0 + a_mb, mblk - 1)) * G + a_kg) * 4096;
+  uint32_t w_off[NTW];
+#pragma unroll
+  for (int t = 0; t < NTW; ++t)
+    w_off[t] = (uint32_t)(min(nbase + 32 * t + (lane >> 1), nseg - 1) * wrow) + 16 * ((lane & 1) ^ ((lane >> 3) & 1));
+  const uint32_t s_off = (uint32_t)min(nbase + lane, nseg - 1) * (2 * G);
+  const uint32_t ring_l = lds_addr(ring);
+  const uint32_t sb_l = lds_addr(sbl_all) + wave * 2048;
+  auto issue = [&](int j, int sl) {
+    const uint32_t dst = ring_l + sl * C::kSlot;
+    dma16x4(a_src + (size_t)j * (WK * 4096), 16 * lane, dst + (a_kg * MTW + a_mb) * 4096);
+    dma16x2(wb + (j * WK + wk) * 32, w_off[0], w_off[1], dst + C::kABytes + (wk * WN + wn) * 2048);
+  };
+
+  f16v y[MTW][NTW];
+#pragma unroll
+  for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NTW; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) y[mt][nt][i] = 0.0f;
+  const NibbleConsts nk = nibble16_consts();
+
+  dma16_unless(0, sb, s_off, sb_l);  // the first 8 groups' scale words
+#pragma unroll
+  for (int j = 0; j < kBigSlots; ++j) issue(min(j, nsteps - 1), j);
+
+  // the bias term first, while the ring fills: y = sum_g (b_g - 16 s_g) sum x_g on MFMA, A =
+  // the sums x of 32 operand rows x 16 groups, each split into three bf16 terms (exact to
+  // about 2^-24 of it), B = the rows' biases and their scales times -16 (exact in bf16); the
+  // wave set wk takes every WK-th 16-group step
+  {
+    uint32_t r_off[NTW];
+#pragma unroll
+    for (int nt = 0; nt < NTW; ++nt) r_off[nt] = (uint32_t)min(nbase + 32 * nt + nn, nseg - 1) * (2 * G) + 16 * h;
+    const int rows = 16 * p.mtiles, nks = G / 16;
+    const float* xs[MTW];
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt)
+      xs[mt] = p.xsum + ((size_t)layer * G + 8 * h) * rows + 32 * min(mb0 + mt, mblk - 1) + nn;
+    float v[MTW][8];
+    u32x4 bs[NTW], bb[NTW];
+    auto fetch = [&](int ks) {
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) {
+        bs[nt] = *reinterpret_cast<const u32x4*>(sb + r_off[nt] + 32 * ks);
+        bb[nt] = *reinterpret_cast<const u32x4*>(bb_ + r_off[nt] + 32 * ks);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[mt][i] = xs[mt][(size_t)(16 * ks + i) * rows];
+    };
+    if (wk < nks) fetch(wk);
+    for (int ks = wk; ks < nks; ks += WK) {
+      bf8 b0[NTW], s0[NTW];
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) {
+        b0[nt] = __builtin_bit_cast(bf8, bb[nt]);
+        u32x4 t;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = -16.0f * __builtin_bit_cast(float, bs[nt][e] << 16);
+          const float hi = -16.0f * __builtin_bit_cast(float, bs[nt][e] & 0xFFFF0000u);
+          t[e] = (__builtin_bit_cast(uint32_t, lo) >> 16) | (__builtin_bit_cast(uint32_t, hi) & 0xFFFF0000u);
+        }
+        s0[nt] = __builtin_bit_cast(bf8, t);
+      }
+      float vc[MTW][8];
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) vc[mt][i] = v[mt][i];
+      fetch(min(ks + WK, nks - 1));
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt) {
+        bf8 x3[3];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float hv = rbf(vc[mt][i]);
+          const float r1 = vc[mt][i] - hv;
+          const float m1 = rbf(r1);
+          x3[0][i] = __builtin_bit_cast(__bf16, (uint16_t)(__builtin_bit_cast(uint32_t, hv) >> 16));
+          x3[1][i] = __builtin_bit_cast(__bf16, (uint16_t)(__builtin_bit_cast(uint32_t, m1) >> 16));
+          x3[2][i] = (__bf16)(r1 - m1);
+        }
+#pragma unroll
+        for (int t = 2; t >= 0; --t)
+#pragma unroll
+          for (int nt = 0; nt < NTW; ++nt) {
+            y[mt][nt] = mfma32(x3[t], b0[nt], y[mt][nt]);
+            y[mt][nt] = mfma32(x3[t], s0[nt], y[mt][nt]);
+          }
+      }
+    }
+  }
+
+  // The loop. A step's 2 MTW tiles in sequence, each tile's FMAs between the next one's MFMAs
+  // (the last tile's in the next step). Left to itself the compiler issues a tile's four MFMAs
+  // and then all its FMAs, so the order is held by schedule barriers. The step's one barrier
+  // stands before its last two tiles, behind which nothing reads the step's slot any more:
+  // there every wave's loads of the next step are done (all but the newest step's are, in each
+  // wave, by its wait), so the last tiles already read the next step's first operands, and the
+  // slot is refilled with the step kBigSlots ahead.
+  constexpr int T = MTW * NTW;
+  static_assert(T >= 4 && NTW == 2, "the operand blocks of a step are read before its last two tiles");
+  bf8 b[NTW][4], a[2][4];
+  float sc[NTW], slast = 0.0f;
+  u32x4 wd[NTW];
+  f16v acc[2] = {f16v{}, f16v{}};  // tile t in acc[t & 1]
+  auto read_a = [&](const unsigned char* slot, int mt, int s) {
+    a[mt & 1][s] = *reinterpret_cast<const bf8*>(slot + ((wk * MTW + mt) * 4 + s) * 1024 + 16 * lane);
+  };
+  auto read_w = [&](const unsigned char* slot, int nt) {
+    wd[nt] = *reinterpret_cast<const u32x4*>(slot + C::kABytes + ((wk * WN + wn) * NTW + nt) * 1024 + 32 * nn +
+                                             16 * (h ^ ((nn >> 2) & 1)));
+  };
+  auto read_s = [&](int j, int nt) {
+    return bf2f(sbl_all[wave * 1024 + ((j / C::kSbStride) & 1) * 512 + ((j * WK + wk) & 7) + (32 * nt + nn) * 8]);
+  };
+  auto add = [&](f16v& yt, const f16v& v, float c, int q) {
+#pragma unroll
+    for (int i = 4 * q; i < 4 * q + 4; ++i) yt[i] = __builtin_fmaf(c, v[i], yt[i]);
+  };
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * C::kPerStep) : "memory");
+#pragma unroll
+  for (int nt = 0; nt < NTW; ++nt) {
+    read_w(ring, nt);
+    sc[nt] = read_s(0, nt);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s) read_a(ring, 0, s);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) b[0][s] = nibbles16_bf16(wd[0][s], nk);
+  int sl = 0;
+  for (int j = 0; j < nsteps; ++j) {
+    const unsigned char* slot = ring + sl * C::kSlot;
+    const int sn = sl == kBigSlots - 1 ? 0 : sl + 1;
+    const unsigned char* next = ring + sn * C::kSlot;
+    float scn[NTW];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int mt = t / NTW, nt = t % NTW;
+      if (t == T - 2) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::kPerStep) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        acc[t & 1] = mfma32(a[mt & 1][s], b[nt][s], s == 0 ? f16v{} : acc[t & 1]);
+        if (t == 0) {
+          add(y[MTW - 1][NTW - 1], acc[(T - 1) & 1], slast, s);
+          b[1][s] = nibbles16_bf16(wd[1][s], nk);
+        } else {
+          add(y[(t - 1) / NTW][(t - 1) % NTW], acc[(t - 1) & 1], sc[(t - 1) % NTW], s);
+        }
+        // LDS reads, at most one a product: the next operand block's over this one's two tiles
+        if (mt + 1 < MTW) {
+          if (s % 2 == 0) read_a(slot, mt + 1, 2 * nt + s / 2);
+        } else if (nt == 0) {
+          if (s < NTW) read_w(next, s);
+          else read_a(next, 0, s - NTW);
+          if (s == 0) {
+            const int blk = min(j / C::kSbStride + 1, nblk - 1);
+            dma16_unless(j & (C::kSbStride - 1), sb + 16 * blk, s_off, sb_l + (blk & 1) * 1024);
+          }
+          if (s == 1) issue(min(j + kBigSlots, nsteps - 1), sl);
+        } else {
+          if (s < NTW) read_a(next, 0, 2 + s);
+          else scn[s - NTW] = read_s(min(j + 1, nsteps - 1), s - NTW);
+          b[0][s] = nibbles16_bf16(wd[0][s], nk);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    slast = sc[NTW - 1];
+#pragma unroll
+    for (int nt = 0; nt < NTW; ++nt) sc[nt] = scn[nt];
+    sl = sn;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) y[MTW - 1][NTW - 1][i] = __builtin_fmaf(slast, acc[(T - 1) & 1][i], y[MTW - 1][NTW - 1][i]);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated loads, before the LDS is used again
+
+  // the wave sets' partial sums, in a fixed order
+  if (WK > 1) {
+    f4* red = reinterpret_cast<f4*>(ring);  // [set - 1][wave of the set][tile][4][64]
+    const int w0 = wn * T * 4 * 64 + lane;
+    constexpr int kSet = WN * T * 4 * 64;
+    __syncthreads();
+    if (wk > 0) {
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f16v& v = y[t / NTW][t % NTW];
+          red[(wk - 1) * kSet + w0 + (t * 4 + i) * 64] = f4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        }
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int q = 0; q < WK - 1; ++q)
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f4 r = red[q * kSet + w0 + (t * 4 + i) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[t / NTW][t % NTW][4 * i + e] += r[e];
+        }
+  }
+#pragma unroll
+  for (int nt = 0; nt < NTW; ++nt) {
+    const int n = nbase + 32 * nt + nn;
+    if (n < nseg) {
+      uint16_t* yr = yseg + (size_t)layer * p.M * nseg + n;
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int m = 32 * (mb0 + mt) + 8 * (i / 4) + 4 * h + (i & 3);
+          if (m < p.M) yr[(size_t)m * nseg] = f2bf(y[mt][nt][i]);
+        }
+    }
+  }
+}
+
 template <bool NORM>
 hipError_t launch_j(int J, const QParams& p, dim3 grid, size_t smem, hipStream_t stream) {
   switch (J) {
@@ -868,14 +1242,97 @@ int qgemm_mtiles(int m) {
   return ((m + 15) / 16 + mt - 1) / mt * mt;
 }
 
-template <int MT>
+template <int MT, bool F32>
 hipError_t launch_gemm_mt(int NT, const QParams& p, dim3 grid, hipStream_t stream) {
   switch (NT) {
-    case 1: hipLaunchKernelGGL((qgemm_kernel<MT, 1>), grid, dim3(kThreads), 0, stream, p); break;
-    case 2: hipLaunchKernelGGL((qgemm_kernel<MT, 2>), grid, dim3(kThreads), 0, stream, p); break;
-    default: hipLaunchKernelGGL((qgemm_kernel<MT, 4>), grid, dim3(kThreads), 0, stream, p); break;
+    case 1: hipLaunchKernelGGL((qgemm_kernel<MT, 1, F32>), grid, dim3(kThreads), 0, stream, p); break;
+    case 2: hipLaunchKernelGGL((qgemm_kernel<MT, 2, F32>), grid, dim3(kThreads), 0, stream, p); break;
+    default: hipLaunchKernelGGL((qgemm_kernel<MT, 4, F32>), grid, dim3(kThreads), 0, stream, p); break;
   }
   return hipGetLastError();
+}
+
+// qgemm_kernel over the p.R rows of p: MT m tiles and NT row tiles per workgroup
+template <bool F32>
+hipError_t launch_gemm(QParams p, int n_layers, int MT, hipStream_t stream) {
+  const int gy = p.mtiles / MT;
+  // weight rows per workgroup: 64, 32 or 16 -- the most that still gives 512 workgroups
+  int NT = 4;
+  while (NT > 1 && (size_t)n_layers * ((p.R + 16 * NT - 1) / (16 * NT)) * gy < 512) NT /= 2;
+  p.tiles = (p.R + 16 * NT - 1) / (16 * NT);
+  p.mgroups = gy;
+  const size_t nwg = (size_t)n_layers * p.tiles * gy;
+  p.remap = (gy > 1 || n_layers >= 8) && nwg % 8 == 0;
+  const dim3 grid((unsigned)nwg);
+  if (F32) return launch_gemm_mt<4, F32>(NT, p, grid, stream);  // (its operand has whole 64-row groups)
+  switch (MT) {
+    case 1: return launch_gemm_mt<1, false>(NT, p, grid, stream);
+    case 2: return launch_gemm_mt<2, false>(NT, p, grid, stream);
+    case 3: return launch_gemm_mt<3, false>(NT, p, grid, stream);
+    default: return launch_gemm_mt<4, false>(NT, p, grid, stream);
+  }
+}
+
+// The weight rows qgemm_big_kernel takes of an n-row matrix, in whole tiles of `rows`; a last
+// partial tile where it is at least 5/8 full.
+int big_tiles(int n, int rows) { return n / rows + (n % rows >= rows * 5 / 8 ? 1 : 0); }
+
+// Workgroups of qgemm_big_kernel<WN, WK, MTW> on the busiest CU, or the whole call's (per_cu = 1)
+template <int WN, int WK, int MTW>
+size_t big_workgroups(const QParams& p, int n_layers, int per_cu) {
+  size_t t = 0;
+  for (int q = 0; q < p.nseg; ++q) t += big_tiles(p.n[q], BigCfg<WN, WK, MTW>::kRows);
+  return (t * n_layers * ((p.mtiles / 2 + MTW - 1) / MTW) + per_cu - 1) / per_cu;
+}
+
+// Which form of the product a call of more than 48 rows takes: 0 qgemm_kernel, 1 the 128 x 256
+// tiles, 2 the 64 x 128 ones (K split in two). Measured at K = 5120 and 6144 (the layer's
+// projections), a CU with n workgroups takes about 85 n + 10 us with the large tiles and
+// 24 n + 24 us with the small ones: in_proj M = 333 109 (large) / 101 us, M = 512 117 / 125,
+// M = 1024 190 / 223, M = 4096 700 / 871; out_proj M = 1024 117 / 107, M = 2048 197 / 181,
+// M = 4096 342 / 349. With few small tiles most CUs stand idle and qgemm_kernel's 64 x 64 tiles
+// split over more workgroups are faster: out_proj M = 128 (80 tiles) 37 us against 45, in_proj
+// M = 64 (128) 47 against 52; from 160 (out_proj M = 256) 47 against 56, in_proj M = 128 (256)
+// 55 against 62.
+int big_form(const QParams& p, int n_layers) {
+  constexpr int kCUs = 256;
+  if (big_workgroups<2, 2, 2>(p, n_layers, 1) < 144) return 0;
+  const size_t large = big_workgroups<4, 1, 4>(p, n_layers, kCUs), small = big_workgroups<2, 2, 2>(p, n_layers, kCUs);
+  return big_workgroups<4, 1, 4>(p, n_layers, 1) > 0 && 85 * large + 10 <= 24 * small + 24 ? 1 : 2;
+}
+
+template <int WN, int WK, int MTW>
+hipError_t launch_big(QParams p, int n_layers, hipStream_t stream) {
+  using C = BigCfg<WN, WK, MTW>;
+  int t = 0;
+  for (int q = 0; q < p.nseg; ++q) {
+    p.row0[q] = t;
+    t += big_tiles(p.n[q], C::kRows);
+  }
+  p.tiles = t;
+  p.mgroups = (p.mtiles / 2 + MTW - 1) / MTW;
+  const size_t nwg = (size_t)n_layers * p.tiles * p.mgroups;
+  p.remap = nwg % 8 == 0;
+  hipLaunchKernelGGL((qgemm_big_kernel<WN, WK, MTW>), dim3((unsigned)nwg), dim3(kThreads), 0, stream, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  // the rows past the whole tiles (in_proj_a and in_proj_b are all such rows)
+  QParams r = p;
+  r.nseg = 0;
+  r.R = 0;
+  for (int q = 0; q < p.nseg; ++q) {
+    const int done = std::min(p.n[q], big_tiles(p.n[q], C::kRows) * C::kRows);
+    if (done == p.n[q]) continue;
+    const int i = r.nseg++;
+    r.w[i] = p.w[q] + (size_t)done * (p.K / 8);
+    r.s[i] = p.s[q] + (size_t)done * (p.K / 64);
+    r.b[i] = p.b[q] + (size_t)done * (p.K / 64);
+    r.y[i] = p.y[q] + done;
+    r.n[i] = p.n[q];
+    r.row0[i] = r.R;
+    r.R += p.n[q] - done;
+  }
+  return r.R ? launch_gemm<true>(r, n_layers, 4, stream) : hipSuccess;
 }
 }  // namespace
 
@@ -959,21 +1416,28 @@ hipError_t launch_qlinear(const gdn_qlinear_args& a, hipStream_t stream) {
   p.mtiles = qgemm_mtiles(a.m);
   p.xfrag = static_cast<uint16_t*>(a.workspace);
   p.xsum = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + qlinear_xfrag_bytes(a.n_layers, a.m, a.k));
+  // qgemm_ns_kernel and qgemm_big_kernel load scales and biases 16 bytes a lane, the latter at
+  // 32-bit offsets in a matrix
+  bool sb16 = true, off32 = true;
+  for (int q = 0; q < a.n_segs; ++q) {
+    sb16 = sb16 && reinterpret_cast<uintptr_t>(a.segs[q].scales) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(a.segs[q].biases) % 16 == 0;
+    off32 = off32 && (size_t)a.segs[q].n * (a.k / 2) <= UINT32_MAX;
+  }
+  const int big = sb16 && off32 && p.mtiles > 3 ? big_form(p, a.n_layers) : 0;
+  p.frag32 = big != 0;
   const size_t prep_threads = (size_t)a.n_layers * 16 * p.mtiles * (a.k / 32) * 4;
   const dim3 gp((unsigned)((prep_threads + kThreads - 1) / kThreads));
   if (norm) hipLaunchKernelGGL(qprep_kernel<true>, gp, dim3(kThreads), 0, stream, p, a.n_layers);
   else hipLaunchKernelGGL(qprep_kernel<false>, gp, dim3(kThreads), 0, stream, p, a.n_layers);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int gy = p.mtiles / MT;
+  if (big == 1) return launch_big<4, 1, 4>(p, a.n_layers, stream);
+  if (big == 2) return launch_big<2, 2, 2>(p, a.n_layers, stream);
+
   // one m group and enough 256-row workgroups for two per CU: the operand-sharing kernel
-  // (its scale and bias loads take 16 bytes a lane)
-  bool sb16 = true;
-  for (int q = 0; q < a.n_segs; ++q)
-    sb16 = sb16 && reinterpret_cast<uintptr_t>(a.segs[q].scales) % 16 == 0 &&
-           reinterpret_cast<uintptr_t>(a.segs[q].biases) % 16 == 0;
   const int ns_tiles = (R + kNsRows - 1) / kNsRows;
-  if (gy == 1 && MT <= 3 && sb16 && (size_t)a.n_layers * ns_tiles >= 512) {
+  if (p.mtiles == MT && MT <= 3 && sb16 && (size_t)a.n_layers * ns_tiles >= 512) {
     p.tiles = ns_tiles;
     p.mgroups = 1;
     const size_t nwg = (size_t)a.n_layers * ns_tiles;
@@ -986,20 +1450,7 @@ hipError_t launch_qlinear(const gdn_qlinear_args& a, hipStream_t stream) {
     }
     return hipGetLastError();
   }
-  // weight rows per workgroup: 64, 32 or 16 -- the most that still gives 512 workgroups
-  int NT = 4;
-  while (NT > 1 && (size_t)a.n_layers * ((R + 16 * NT - 1) / (16 * NT)) * gy < 512) NT /= 2;
-  p.tiles = (R + 16 * NT - 1) / (16 * NT);
-  p.mgroups = gy;
-  const size_t nwg = (size_t)a.n_layers * p.tiles * gy;
-  p.remap = (gy > 1 || a.n_layers >= 8) && nwg % 8 == 0;
-  const dim3 grid((unsigned)nwg);
-  switch (MT) {
-    case 1: return launch_gemm_mt<1>(NT, p, grid, stream);
-    case 2: return launch_gemm_mt<2>(NT, p, grid, stream);
-    case 3: return launch_gemm_mt<3>(NT, p, grid, stream);
-    default: return launch_gemm_mt<4>(NT, p, grid, stream);
-  }
+  return launch_gemm<false>(p, a.n_layers, MT, stream);
 }
 
 }  // namespace gdn

@@ -406,3 +406,36 @@ def test_qlinear_4096_rows_two_layers(O, gdn, dev):
     got = to_np(y)
     for l in range(L):
         check(got[l], O.qlinear_blocked(x[l], w[l], s[l], b[l]), bound(O, x[l], s[l], b[l]), f"layer {l}")
+
+
+# ---- the LDS-tiled product (qgemm_big_kernel) ----
+# Calls of more than 48 rows and at least 144 tiles of 64 operand x 128 weight rows take it, in
+# tiles of 64 x 128 or (few enough workgroups a CU, see big_form) 128 x 256. A matrix's rows past
+# its whole tiles are a partial tile where it is 5/8 full, else qgemm_kernel's.
+
+@pytest.mark.parametrize("L,M,K,ns", [
+    (1, 129, 1024, [6200, 100, 48]),   # 64 x 128: 48 tiles + 56 rows, a partial tile, a matrix of leftovers only
+    (2, 65, 2048, [5000]),             # two layers, one operand row in the second 64
+    (1, 260, 8192, [4096 + 7]),        # the longest K, seven leftover rows
+    (1, 1000, 1024, [8000, 200, 24]),  # 128 x 256: 31 tiles + 64 rows, a partial tile, leftovers only
+    (1, 897, 5120, [8192 + 255]),      # a partial tile of 255 rows; one row in the last 128
+])
+def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
+    import torch
+    log_case(f"qlinear (LDS tiles) L={L} M={M} K={K} N={ns}")
+    rng = np.random.default_rng(M + K)
+    mats, host, x = [], [], None
+    for i, n in enumerate(ns):
+        xi, w, s, b = quant_inputs(O, L, M, n, K, seed=M + K + i)
+        x = xi if x is None else x
+        mats.append(dev_mat(gdn, dev, w, s, b) if L > 1 else dev_mat(gdn, dev, w[0], s[0], b[0]))
+        host.append((w, s, b))
+    ys = gdn.qlinear(mats, to_dev(x if L > 1 else x[0], dev), n_layers=L)
+    torch.cuda.synchronize()
+    for i, ((w, s, b), y) in enumerate(zip(host, ys)):
+        got = to_np(y).reshape(L, M, -1)
+        n = w.shape[1]
+        rows = sampled_rows(n, rng) if n > 1024 else np.arange(n)
+        for l in range(L):
+            check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], s[l][rows], b[l][rows]),
+                  bound(O, x[l], s[l][rows], b[l][rows]), f"segment {i} layer {l}")
