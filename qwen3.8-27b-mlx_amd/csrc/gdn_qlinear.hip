@@ -909,8 +909,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_ns_kernel(QParams p) {
 // through a ring of kBigSlots LDS slots filled by direct-to-LDS loads ahead of their use; each
 // wave's scale words come 8 groups at a time into its own pair of buffers. Per group and
 // 32 x 32 tile: four products into acc = sum x (16 + q), then y += s acc (16 FMAs a lane
-// beside 128 cycles of MFMA); the bias term is made before the loop on MFMA, as
-// qgemm_ns_kernel does after its. Nibble q is the bf16 16 + q here (q in the mantissa's upper
+// beside 128 cycles of MFMA); the bias term is made on MFMA, as qgemm_ns_kernel does. Nibble q is the bf16 16 + q here (q in the mantissa's upper
 // four bits: one shift more per word than 128 + q): the terms of the offset are summed apart
 // from the products that cancel them, so their size is what the fp32 sums round at, and with
 // 128 the outputs lay further from the exact product than qgemm_kernel's, which cancels them
@@ -994,7 +993,7 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
   const size_t wrow = (size_t)p.K / 2;                 // bytes of a weight row
   const char* const wb = reinterpret_cast<const char*>(wseg) + (size_t)layer * nseg * wrow;
   const char* const sb = reinterpret_cast<const char*>(sseg) + (size_t)layer * nseg * (2 * G);
-  const char* const bb_ = reinterpret_cast<const char*>(bseg) + (size_t)layer * nseg * (2 * G);
+  const char* const bb = reinterpret_cast<const char*>(bseg) + (size_t)layer * nseg * (2 * G);
 
   // this wave's loads of a step: the four blocks of one (group, operand block) and the nibble
   // words of its own 64 rows and group in two loads of 32 rows, a lane pair the 32 bytes of a
@@ -1029,73 +1028,91 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
 #pragma unroll
   for (int j = 0; j < kBigSlots; ++j) issue(min(j, nsteps - 1), j);
 
-  // the bias term first, while the ring fills: y = sum_g (b_g - 16 s_g) sum x_g on MFMA, A =
-  // the sums x of 32 operand rows x 16 groups, each split into three bf16 terms (exact to
-  // about 2^-24 of it), B = the rows' biases and their scales times -16 (exact in bf16); the
-  // wave set wk takes every WK-th 16-group step
-  {
-    uint32_t r_off[NTW];
-#pragma unroll
-    for (int nt = 0; nt < NTW; ++nt) r_off[nt] = (uint32_t)min(nbase + 32 * nt + nn, nseg - 1) * (2 * G) + 16 * h;
-    const int rows = 16 * p.mtiles, nks = G / 16;
-    const float* xs[MTW];
-#pragma unroll
-    for (int mt = 0; mt < MTW; ++mt)
-      xs[mt] = p.xsum + ((size_t)layer * G + 8 * h) * rows + 32 * min(mb0 + mt, mblk - 1) + nn;
+  // The bias term sum_g (b_g - 16 s_g) sum x_g, 16 groups at a time: y += on MFMA, A = the sums x
+  // of 32 operand rows x 16 groups, each split into three bf16 terms (exact to about 2^-24 of
+  // it), B = the rows' biases and their scales times -16 (exact in bf16). The large tiles (all
+  // of K in one sum) add a block's term just before its groups' products, which cancel most of
+  // it, so that y stays near its final size: with the whole term first, the share of in_proj
+  // outputs off the exact product's rounding was 1.0e-3 instead of 0.5e-3 (qgemm_kernel:
+  // 1.2e-3). With K split, the wave set wk adds every WK-th block first, while the ring fills:
+  // 4 us less at M = 333 (out_proj: 2.4e-3 to 3.1e-3 off, qgemm_kernel 2.9e-3 to 3.6e-3).
+  const int rows = 16 * p.mtiles, nks = G / 16;
+  const float* const xs0 = p.xsum + (size_t)layer * G * rows;
+  struct BiasBlock {
+    u32x4 s[NTW], b[NTW];
     float v[MTW][8];
-    u32x4 bs[NTW], bb[NTW];
-    auto fetch = [&](int ks) {
+  };
+  // the lane, opaque: the addresses below are made from it at each use and hold no registers in
+  // the loop
+  auto opaque_lane = [&]() {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  auto load_rows = [&](int ks, int l, BiasBlock& q) {
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt) {
-        bs[nt] = *reinterpret_cast<const u32x4*>(sb + r_off[nt] + 32 * ks);
-        bb[nt] = *reinterpret_cast<const u32x4*>(bb_ + r_off[nt] + 32 * ks);
+    for (int nt = 0; nt < NTW; ++nt) {
+      const uint32_t off = (uint32_t)min(nbase + 32 * nt + (l & 31), nseg - 1) * (2 * G) + 16 * (l >> 5) + 32 * ks;
+      q.s[nt] = *reinterpret_cast<const u32x4*>(sb + off);
+      q.b[nt] = *reinterpret_cast<const u32x4*>(bb + off);
+    }
+  };
+  auto load_sums = [&](int ks, int l, int mt, BiasBlock& q) {
+    const uint32_t off = (uint32_t)(16 * ks + 8 * (l >> 5)) * rows + 32 * min(mb0 + mt, mblk - 1) + (l & 31);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q.v[mt][i] = xs0[off + (uint32_t)(i * rows)];
+  };
+  // (inside the loop the sums are loaded here, an operand block at a time: no registers for all
+  // of them beside the loop's)
+  auto add_bias = [&](BiasBlock& q, int ks, int l) {
+    bf8 b0[NTW], s0[NTW];
+#pragma unroll
+    for (int nt = 0; nt < NTW; ++nt) {
+      b0[nt] = __builtin_bit_cast(bf8, q.b[nt]);
+      u32x4 t;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = -16.0f * __builtin_bit_cast(float, q.s[nt][e] << 16);
+        const float hi = -16.0f * __builtin_bit_cast(float, q.s[nt][e] & 0xFFFF0000u);
+        t[e] = (__builtin_bit_cast(uint32_t, lo) >> 16) | (__builtin_bit_cast(uint32_t, hi) & 0xFFFF0000u);
+      }
+      s0[nt] = __builtin_bit_cast(bf8, t);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) {
+      if (WK == 1) load_sums(ks, l, mt, q);
+      bf8 x3[3];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float hv = rbf(q.v[mt][i]);
+        const float r1 = q.v[mt][i] - hv;
+        const float m1 = rbf(r1);
+        x3[0][i] = __builtin_bit_cast(__bf16, (uint16_t)(__builtin_bit_cast(uint32_t, hv) >> 16));
+        x3[1][i] = __builtin_bit_cast(__bf16, (uint16_t)(__builtin_bit_cast(uint32_t, m1) >> 16));
+        x3[2][i] = (__bf16)(r1 - m1);
       }
 #pragma unroll
-      for (int mt = 0; mt < MTW; ++mt)
+      for (int t = 2; t >= 0; --t)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[mt][i] = xs[mt][(size_t)(16 * ks + i) * rows];
+        for (int nt = 0; nt < NTW; ++nt) {
+          y[mt][nt] = mfma32(x3[t], b0[nt], y[mt][nt]);
+          y[mt][nt] = mfma32(x3[t], s0[nt], y[mt][nt]);
+        }
+      if (WK == 1 && mt % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (WK > 1 && wk < nks) {
+    BiasBlock q;
+    auto load = [&](int ks) {
+      load_rows(ks, lane, q);
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt) load_sums(ks, lane, mt, q);
     };
-    if (wk < nks) fetch(wk);
+    load(wk);
     for (int ks = wk; ks < nks; ks += WK) {
-      bf8 b0[NTW], s0[NTW];
-#pragma unroll
-      for (int nt = 0; nt < NTW; ++nt) {
-        b0[nt] = __builtin_bit_cast(bf8, bb[nt]);
-        u32x4 t;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float lo = -16.0f * __builtin_bit_cast(float, bs[nt][e] << 16);
-          const float hi = -16.0f * __builtin_bit_cast(float, bs[nt][e] & 0xFFFF0000u);
-          t[e] = (__builtin_bit_cast(uint32_t, lo) >> 16) | (__builtin_bit_cast(uint32_t, hi) & 0xFFFF0000u);
-        }
-        s0[nt] = __builtin_bit_cast(bf8, t);
-      }
-      float vc[MTW][8];
-#pragma unroll
-      for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) vc[mt][i] = v[mt][i];
-      fetch(min(ks + WK, nks - 1));
-#pragma unroll
-      for (int mt = 0; mt < MTW; ++mt) {
-        bf8 x3[3];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float hv = rbf(vc[mt][i]);
-          const float r1 = vc[mt][i] - hv;
-          const float m1 = rbf(r1);
-          x3[0][i] = __builtin_bit_cast(__bf16, (uint16_t)(__builtin_bit_cast(uint32_t, hv) >> 16));
-          x3[1][i] = __builtin_bit_cast(__bf16, (uint16_t)(__builtin_bit_cast(uint32_t, m1) >> 16));
-          x3[2][i] = (__bf16)(r1 - m1);
-        }
-#pragma unroll
-        for (int t = 2; t >= 0; --t)
-#pragma unroll
-          for (int nt = 0; nt < NTW; ++nt) {
-            y[mt][nt] = mfma32(x3[t], b0[nt], y[mt][nt]);
-            y[mt][nt] = mfma32(x3[t], s0[nt], y[mt][nt]);
-          }
-      }
+      BiasBlock c = q;
+      load(min(ks + WK, nks - 1));
+      add_bias(c, ks, lane);
     }
   }
 
@@ -1137,7 +1154,15 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
 #pragma unroll
   for (int s = 0; s < 4; ++s) b[0][s] = nibbles16_bf16(wd[0][s], nk);
   int sl = 0;
-  for (int j = 0; j < nsteps; ++j) {
+  constexpr int kSpan = WK == 1 ? 16 : 8;  // steps (nsteps is a multiple of it) between bias blocks, if any
+  for (int j0 = 0; j0 < nsteps; j0 += kSpan) {
+  if (WK == 1) {
+    BiasBlock q;
+    const int l = opaque_lane();
+    load_rows(j0 / kSpan, l, q);
+    add_bias(q, j0 / kSpan, l);
+  }
+  for (int j = j0; j < j0 + kSpan; ++j) {
     const unsigned char* slot = ring + sl * C::kSlot;
     const int sn = sl == kBigSlots - 1 ? 0 : sl + 1;
     const unsigned char* next = ring + sn * C::kSlot;
@@ -1181,6 +1206,7 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) sc[nt] = scn[nt];
     sl = sn;
+  }
   }
 #pragma unroll
   for (int i = 0; i < 16; ++i) y[MTW - 1][NTW - 1][i] = __builtin_fmaf(slast, acc[(T - 1) & 1][i], y[MTW - 1][NTW - 1][i]);
