@@ -8,8 +8,8 @@
 // out_proj, so norm and projection are one launch.
 //
 // HBM-bound at decode (M = B * L rows of x, 1..4): every weight byte is read once.
-// Mapping: a workgroup stages its operand in LDS, then each wave takes 4 output rows at a
-// time, one per 16-lane DPP row; lane m of a row reads the row's 16-byte pieces m, m + 16,
+// Mapping: a workgroup of 4 or 8 waves stages its operand in LDS, then each wave takes 4 output
+// rows at a time, one per 16-lane DPP row; lane m of a row reads the row's 16-byte pieces m, m + 16,
 // m + 32, ... (each 32 nibbles = half a group), so a load instruction reads 4 x 256
 // contiguous bytes; the rows' scale and bias words come 16 bytes a lane, ahead of the
 // weights, and reach the lanes that use them through the wave's LDS rows. A nibble v becomes the bf16 value 128 + v with one and-or
@@ -47,10 +47,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // global-memory pointers: a plain pointer that passed through a struct can lose its
 // address space and compile to flat loads, which also count against the LDS wait counter
 typedef const u32x2 __attribute__((address_space(1))) g_u32x2;
-typedef const uint16_t __attribute__((address_space(1))) g_u16;
+typedef const u32x4 __attribute__((address_space(1))) g_u32x4;
 
 constexpr int kThreads = 256;
-constexpr int kRowsPerPass = 16;  // 4 waves x 4 DPP rows
 
 struct QParams {
   int M, K, R, tiles, nseg;
@@ -91,10 +90,18 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
   return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
 }
 
-// Operand chunk (32 values) to LDS: four 16-byte words, word i holding the pairs
-// (v[8i+j], v[8i+j+4]), j = 0..3, the order the nibble pairs come out in; plus the sum
-// of the 32 values.
-__device__ __forceinline__ void stage_chunk(u32x4* xs, float* xsum, int nch, int mm, int c, const float (&v)[32]) {
+// Operand chunk c (32 values) of row mm to LDS: four 16-byte words, word i holding the pairs
+// (v[8i+j], v[8i+j+4]), j = 0..3, the order the nibble pairs come out in; plus the sum of the
+// 32 values.
+__device__ __forceinline__ void stage_chunk(const QParams& p, u32x4* xs, float* xsum, int nch, int layer, int mm, int c) {
+  const uint16_t* src = p.x + ((size_t)layer * p.M + mm) * p.K + 32 * c;
+  float v[32];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const u16x8 xx = *reinterpret_cast<const u16x8*>(src + 8 * q);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[8 * q + e] = bf2f(xx[e]);
+  }
   float sum = 0.0f;
 #pragma unroll
   for (int e = 0; e < 32; ++e) sum += v[e];
@@ -108,47 +115,32 @@ __device__ __forceinline__ void stage_chunk(u32x4* xs, float* xsum, int nch, int
   xsum[mm * nch + c] = sum;
 }
 
-// The operand of row mrow, values 32 c .. 32 c + 31, into v: x as given, or the GatedRMSNorm
-// of (xf, z) (the four pieces of a 128-value head are the lanes of a DPP quad).
-template <bool NORM>
-__device__ __forceinline__ void operand_piece(const QParams& p, int layer, int mrow, int c, float (&v)[32]) {
-  const size_t base = ((size_t)layer * p.M + mrow) * p.K + 32 * c;
-  if (NORM) {
-    // GatedRMSNorm: h = o * rsqrt(mean(o^2) + eps) * gamma (fp32), times silu(fp32(z)),
-    // rounded to bf16 (the activation dtype out_proj takes)
-    float o[32];
+// The GatedRMSNorm of (xf, z) (model.cpp:350-354) as the operand: h = o * rsqrt(mean(o^2) +
+// eps) * gamma (fp32), times silu(fp32(z)), rounded to bf16 (the activation dtype out_proj
+// takes). A lane takes 8 values; the 16 lanes of a DPP row hold a 128-value head, whose sum of
+// squares is 8 terms a lane and a row sum.
+struct NormIn {
+  f4 o[2];
+  u16x8 z;
+};
+__device__ __forceinline__ NormIn norm_load(const QParams& p, size_t at) {
+  NormIn n;
+  n.o[0] = *reinterpret_cast<const f4*>(p.xf + at);
+  n.o[1] = *reinterpret_cast<const f4*>(p.xf + at + 4);
+  n.z = *reinterpret_cast<const u16x8*>(p.z + at);
+  return n;
+}
+__device__ __forceinline__ void gated_rmsnorm8(const NormIn& n, const f4 (&gm)[2], float eps, float (&v)[8]) {
+  float ss = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const f4 f = *reinterpret_cast<const f4*>(p.xf + base + 4 * q);
+  for (int e = 0; e < 8; ++e) ss += n.o[e / 4][e % 4] * n.o[e / 4][e % 4];
+  ss = row16_sum(ss);
+  const float rs = 1.0f / sqrtf(ss / 128.0f + eps);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[4 * q + e] = f[e];
-    }
-    float ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 32; ++e) ss += o[e] * o[e];
-    ss += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, ss), 0xB1, 0xF, 0xF, true));
-    ss += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, ss), 0x4E, 0xF, 0xF, true));
-    const float rs = 1.0f / sqrtf(ss / 128.0f + p.eps);
-    const float* gm = p.gamma + (size_t)layer * 128 + 32 * (c & 3);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const u16x8 zz = *reinterpret_cast<const u16x8*>(p.z + base + 8 * q);
-      const f4 g0 = *reinterpret_cast<const f4*>(gm + 8 * q);
-      const f4 g1 = *reinterpret_cast<const f4*>(gm + 8 * q + 4);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float zf = bf2f(zz[e]);
-        const float h = o[8 * q + e] * rs * (e < 4 ? g0[e] : g1[e - 4]);
-        v[8 * q + e] = rbf(h * (zf * d_sigmoidf(zf)));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const u16x8 xx = *reinterpret_cast<const u16x8*>(p.x + base + 8 * q);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[8 * q + e] = bf2f(xx[e]);
-    }
+  for (int e = 0; e < 8; ++e) {
+    const float zf = bf2f(n.z[e]);
+    const float h = n.o[e / 4][e % 4] * rs * gm[e / 4][e % 4];
+    v[e] = rbf(h * (zf * d_sigmoidf(zf)));
   }
 }
 
@@ -167,212 +159,6 @@ __device__ __forceinline__ NibbleConsts nibble_consts() {
   k.bias = 0x43004300u;
   asm volatile("" : "+v"(k.mask), "+v"(k.bias));  // (emits nothing: keeps them opaque VGPR values)
   return k;
-}
-
-template <int J, bool NORM>
-__global__ __launch_bounds__(kThreads) void qlinear_kernel(QParams p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  // each wave's scale and bias words of its current 4 rows: [wave][row][scale, bias][group]
-  __shared__ __attribute__((aligned(16))) uint16_t sbs[4][4][2][8192 / 64];
-  const int layer = blockIdx.x / p.tiles;
-  const int tile = blockIdx.x % p.tiles;
-  const int K = J * 512, nch = K / 32;
-  u32x4* xs = reinterpret_cast<u32x4*>(smem);                 // [M][4][nch]
-  float* xsum = reinterpret_cast<float*>(xs + p.M * 4 * nch);  // [M][nch]
-  const int tid = threadIdx.x;
-
-  // ---- stage the operand: thread task t = (row mm, chunk c); the four chunks of a
-  // 128-value head are the four lanes of a DPP quad ----
-  for (int t = tid; t < p.M * nch; t += kThreads) {
-    const int mm = t / nch, c = t % nch;
-    float v[32];
-    operand_piece<NORM>(p, layer, mm, c, v);
-    stage_chunk(xs, xsum, nch, mm, c, v);
-  }
-  __syncthreads();
-
-  // ---- passes of 4 rows per wave ----
-  const NibbleConsts nk = nibble_consts();
-  const int lane = tid & 63, m = lane & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int passes = p.passes;
-  for (int pass = 0; pass < passes; ++pass) {
-    const int grow = (tile * passes + pass) * kRowsPerPass + wave * 4 + (lane >> 4);
-    const bool valid = grow < p.R;
-    const int row = valid ? grow : p.R - 1;
-    int sg = 0;
-#pragma unroll
-    for (int q = 1; q < GDN_QLINEAR_MAX_SEGS; ++q) sg += (q < p.nseg && row >= p.row0[q]) ? 1 : 0;
-    const uint32_t* wseg = p.w[0];
-    const uint16_t *sseg = p.s[0], *bseg = p.b[0];
-    uint16_t* yseg = p.y[0];
-    int nseg = p.n[0], r0 = p.row0[0];
-#pragma unroll
-    for (int q = 1; q < GDN_QLINEAR_MAX_SEGS; ++q) {
-      if (sg == q) {
-        wseg = p.w[q];
-        sseg = p.s[q];
-        bseg = p.b[q];
-        yseg = p.y[q];
-        nseg = p.n[q];
-        r0 = p.row0[q];
-      }
-    }
-    const size_t lrow = (size_t)layer * nseg + (row - r0);
-    const u32x4* wr = reinterpret_cast<const u32x4*>(wseg + lrow * (K / 8));
-    const uint16_t* sr = sseg + lrow * (K / 64);
-    const uint16_t* br = bseg + lrow * (K / 64);
-    // the row's scale and bias words, 16 bytes a lane (groups 8 mc .. + 7; lanes past the
-    // row's K / 512 chunks repeat the last), first: they arrive before the weights
-    const int mc = m < J ? m : J - 1;
-    const u32x4 swd = *reinterpret_cast<const u32x4*>(sr + 8 * mc);
-    const u32x4 bwd = *reinterpret_cast<const u32x4*>(br + 8 * mc);
-    u32x4 wv[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) wv[j] = __builtin_nontemporal_load(wr + m + 16 * j);
-    // through this wave's LDS rows (written and read by this wave only: no barrier) to the
-    // lanes that use them: piece m + 16 j is in group m / 2 + 8 j
-    uint16_t* srl = &sbs[wave][lane >> 4][0][0];
-    uint16_t* brl = &sbs[wave][lane >> 4][1][0];
-    *reinterpret_cast<u32x4*>(srl + 8 * mc) = swd;
-    *reinterpret_cast<u32x4*>(brl + 8 * mc) = bwd;
-    float y[GDN_QLINEAR_GEMV_ROWS] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int c = m + 16 * j;
-      const float sc = bf2f(srl[(m >> 1) + 8 * j]);
-      const float off = bf2f(brl[(m >> 1) + 8 * j]) - 128.0f * sc;
-      uint32_t pr[4][4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t wd = wv[j][i];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) pr[i][q] = and_or(wd >> (4 * q), nk.mask, nk.bias);
-      }
-#pragma unroll
-      for (int mm = 0; mm < GDN_QLINEAR_GEMV_ROWS; ++mm) {
-        if (mm < p.M) {
-          float acc = 0.0f;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const u32x4 xq = xs[(mm * 4 + i) * nch + c];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc = dot2(pr[i][q], xq[q], acc);
-          }
-          y[mm] = __builtin_fmaf(sc, acc, __builtin_fmaf(off, xsum[mm * nch + c], y[mm]));
-        }
-      }
-    }
-#pragma unroll
-    for (int mm = 0; mm < GDN_QLINEAR_GEMV_ROWS; ++mm) {
-      if (mm < p.M) {
-        const float tot = row16_sum(y[mm]);
-        if (m == 0 && valid) yseg[((size_t)layer * p.M + mm) * nseg + (row - r0)] = f2bf(tot);
-      }
-    }
-  }
-}
-
-// MFMA path, step 1: the operand (normalised when NORM) into the workspace's fragment
-// order. Workgroup = 16 rows x 256 values of a layer (K / 256 fastest, then row tiles); thread
-// (r, j) takes the 8 values 8 j of each of the two 128-value heads of row r, so a 16-lane DPP
-// row holds one head of one row and reads its contiguous bytes, and the head's sum of squares
-// is 8 terms per thread and a row sum. The 8 KB pass through LDS and leave in the workspace's
-// order, 256 bytes or more at a time. (One thread per 8 values storing its own 16 bytes, its
-// place found with 64-bit divisions, took 47-49 us for in_proj's 4096 rows, 14 us for 1024.)
-template <bool NORM>
-__global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p) {
-  __shared__ __attribute__((aligned(16))) u32x4 tile[512 + 512 / 16];  // 16 bytes of padding every 256
-  const int nch = p.K / 32, rows = 16 * p.mtiles;
-  const int npc = p.K / 256, piece = blockIdx.x % npc, mtl = blockIdx.x / npc;
-  const int mtile = mtl % p.mtiles, layer = mtl / p.mtiles;
-  const int r = threadIdx.x >> 4, j = threadIdx.x & 15;
-  const int mrow = 16 * mtile + r;
-  const bool live = mrow < p.M;
-  const size_t base = ((size_t)layer * p.M + (live ? mrow : 0)) * p.K + 256 * piece + 8 * j;
-  f4 o[2][2], gm[2];
-  u16x8 in[2];  // z with the norm, x without
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-    if (NORM) {
-      o[hh][0] = *reinterpret_cast<const f4*>(p.xf + base + 128 * hh);
-      o[hh][1] = *reinterpret_cast<const f4*>(p.xf + base + 128 * hh + 4);
-    }
-    in[hh] = *reinterpret_cast<const u16x8*>((NORM ? p.z : p.x) + base + 128 * hh);
-  }
-  if (NORM) {
-    const float* g = p.gamma + (size_t)layer * 128 + 8 * j;
-    gm[0] = *reinterpret_cast<const f4*>(g);
-    gm[1] = *reinterpret_cast<const f4*>(g + 4);
-  }
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-    float v[8];
-    if (NORM) {
-      // GatedRMSNorm (model.cpp:350-354): h = o * rsqrt(mean(o^2) + eps) * gamma (fp32), times
-      // silu(fp32(z)), rounded to bf16 (the activation dtype out_proj takes)
-      float ss = 0.0f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += o[hh][e / 4][e % 4] * o[hh][e / 4][e % 4];
-      ss = row16_sum(ss);
-      const float rs = 1.0f / sqrtf(ss / 128.0f + p.eps);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float zf = bf2f(in[hh][e]);
-        const float hv = o[hh][e / 4][e % 4] * rs * gm[e / 4][e % 4];
-        v[e] = live ? rbf(hv * (zf * d_sigmoidf(zf))) : 0.0f;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = live ? bf2f(in[hh][e]) : 0.0f;
-    }
-    u32x4 q;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) q[e] = pack_bf2(v[e], v[e + 4]);
-    // its place among the workgroup's 512 16-byte pieces: 32-value piece c of the 256, quarter
-    // jq of it
-    const int c = 4 * hh + (j >> 2), jq = j & 3;
-    const int at = p.frag32 ? (8 * (c >> 1) + 2 * jq + (c & 1)) * 16 + r
-                            : (2 * (c >> 1) + (jq & 1)) * 64 + 16 * (2 * (c & 1) + (jq >> 1)) + r;
-    tile[at + (at >> 4)] = q;
-    // the group's sum x: the 64 values of (row, group) are the 8 values of each of 8
-    // consecutive threads, added in a fixed order (each thread's 8 in sequence, then a
-    // butterfly over the 8 threads)
-    float sx = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sx += v[e];
-    sx += __shfl_xor(sx, 1, 8);
-    sx += __shfl_xor(sx, 2, 8);
-    sx += __shfl_xor(sx, 4, 8);
-    if ((j & 7) == 0)
-      p.xsum[((size_t)layer * (p.K / 64) + 4 * piece + 2 * hh + (j >> 3)) * rows + mrow] = sx;
-  }
-  __syncthreads();
-  u32x4* out = reinterpret_cast<u32x4*>(p.xfrag);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int at = 256 * i + threadIdx.x;
-    const u32x4 q = tile[at + (at >> 4)];
-    if (p.frag32) {
-      const int run = at >> 4;  // 16 rows of (group, block, half): 256 bytes
-      out[((size_t)layer * (p.mtiles / 2) + mtile / 2) * nch * 128 + (size_t)piece * 1024 + (run >> 1) * 64 +
-          (run & 1) * 32 + (mtile & 1) * 16 + (at & 15)] = q;
-    } else {
-      out[((size_t)layer * p.mtiles + mtile) * nch * 64 + (size_t)piece * 512 + at] = q;
-    }
-  }
-}
-
-__device__ __forceinline__ f4 mfma(bf8 a, bf8 b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// A nibble word (values k .. k + 7) as a B fragment: bf16 128 + v, pairs (i, i + 4).
-__device__ __forceinline__ bf8 nibbles_bf16(uint32_t wd, NibbleConsts k) {
-  u32x4 r;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) r[q] = and_or(wd >> (4 * q), k.mask, k.bias);
-  return __builtin_bit_cast(bf8, r);
 }
 
 // A weight row's segment: its nibble words, scales, biases and output column. Every
@@ -427,6 +213,220 @@ __device__ __forceinline__ RowPtrs row_ptrs(const QParams& p, int layer, int row
   r.y = yseg + (size_t)layer * p.M * nseg + (row - r0);
   r.ystride = nseg;
   return r;
+}
+
+// W waves. NM: the operand's rows, 1 (no branch between the pieces' products) or up to
+// GDN_QLINEAR_GEMV_ROWS.
+template <int J, bool NORM, int W, int NM>
+__global__ __launch_bounds__(64 * W) void qlinear_kernel(QParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  // each wave's scale and bias words of its current 4 rows: [wave][row][scale, bias][group]
+  __shared__ __attribute__((aligned(16))) uint16_t sbs[W][4][2][J * 8];
+  const int layer = blockIdx.x / p.tiles;
+  const int tile = blockIdx.x % p.tiles;
+  constexpr int K = J * 512, nch = K / 32;
+  u32x4* xs = reinterpret_cast<u32x4*>(smem);                 // [M][4][nch]
+  float* xsum = reinterpret_cast<float*>(xs + p.M * 4 * nch);  // [M][nch]
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, m = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int passes = p.passes;
+
+  // a pass's rows: the lane's row and the words it loads of it -- the scale and bias words, 16
+  // bytes a lane (groups 8 mc .. + 7; lanes past the row's K / 512 chunks repeat the last),
+  // first: they arrive before the weights
+  struct Row {
+    uint16_t* y;
+    int ystride;
+    bool valid;
+    u32x4 s, b, w[J];
+  };
+  const int mc = m < J ? m : J - 1;
+  auto load = [&](int pass, Row& r) {
+    const int grow = (tile * passes + pass) * (4 * W) + wave * 4 + (lane >> 4);
+    r.valid = grow < p.R;
+    const int row = r.valid ? grow : p.R - 1;
+    const RowPtrs rp = row_ptrs(p, layer, row);
+    g_u32x4* wr = (g_u32x4*)rp.w;
+    r.s = *(g_u32x4*)(rp.s + 8 * mc);
+    r.b = *(g_u32x4*)(rp.b + 8 * mc);
+#pragma unroll
+    for (int j = 0; j < J; ++j) r.w[j] = __builtin_nontemporal_load(wr + m + 16 * j);
+    r.y = rp.y;
+    r.ystride = rp.ystride;
+  };
+
+  // ---- stage the operand ----
+  if (NORM) {
+    // a wave's 64 pieces of 8 values are 4 heads; a row's J of them go to the waves in turn,
+    // their loads issued ahead of the arithmetic. Piece q is word q % 4 of chunk q / 4.
+    constexpr int kMine = (J + W - 1) / W;
+    const float* g = p.gamma + (size_t)layer * 128 + 8 * m;
+    const f4 gm[2] = {*reinterpret_cast<const f4*>(g), *reinterpret_cast<const f4*>(g + 4)};
+    for (int mm = 0; mm < p.M; ++mm) {
+      const size_t base = ((size_t)layer * p.M + mm) * K + 8 * lane;
+      NormIn in[kMine];
+#pragma unroll
+      for (int i = 0; i < kMine; ++i) in[i] = norm_load(p, base + 512 * min(wave + W * i, J - 1));
+#pragma unroll
+      for (int i = 0; i < kMine; ++i) {
+        if (wave + W * i >= J) break;
+        const int q = 64 * (wave + W * i) + lane;
+        float v[8];
+        gated_rmsnorm8(in[i], gm, p.eps, v);
+        u32x4 wd;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wd[e] = pack_bf2(v[e], v[e + 4]);
+        xs[(mm * 4 + (q & 3)) * nch + (q >> 2)] = wd;
+        float sum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += v[e];
+        sum += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0xB1, 0xF, 0xF, true));
+        sum += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0x4E, 0xF, 0xF, true));
+        if ((q & 3) == 0) xsum[mm * nch + (q >> 2)] = sum;
+      }
+    }
+  } else {
+    for (int t = tid; t < p.M * nch; t += 64 * W) stage_chunk(p, xs, xsum, nch, layer, t / nch, t % nch);
+  }
+  __syncthreads();
+
+  // ---- passes of 4 rows per wave ----
+  const NibbleConsts nk = nibble_consts();
+  for (int pass = 0; pass < passes; ++pass) {
+    Row r;
+    load(pass, r);
+    // through this wave's LDS rows (written and read by this wave only: no barrier) to the
+    // lanes that use them: piece m + 16 j is in group m / 2 + 8 j
+    uint16_t* srl = &sbs[wave][lane >> 4][0][0];
+    uint16_t* brl = &sbs[wave][lane >> 4][1][0];
+    *reinterpret_cast<u32x4*>(srl + 8 * mc) = r.s;
+    *reinterpret_cast<u32x4*>(brl + 8 * mc) = r.b;
+    float y[NM] = {};
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int c = m + 16 * j;
+      const float sc = bf2f(srl[(m >> 1) + 8 * j]);
+      const float off = bf2f(brl[(m >> 1) + 8 * j]) - 128.0f * sc;
+      uint32_t pr[4][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t wd = r.w[j][i];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pr[i][q] = and_or(wd >> (4 * q), nk.mask, nk.bias);
+      }
+#pragma unroll
+      for (int mm = 0; mm < NM; ++mm) {
+        if (NM == 1 || mm < p.M) {
+          float acc = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const u32x4 xq = xs[(mm * 4 + i) * nch + c];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc = dot2(pr[i][q], xq[q], acc);
+          }
+          y[mm] = __builtin_fmaf(sc, acc, __builtin_fmaf(off, xsum[mm * nch + c], y[mm]));
+        }
+      }
+    }
+#pragma unroll
+    for (int mm = 0; mm < NM; ++mm) {
+      if (NM == 1 || mm < p.M) {
+        const float tot = row16_sum(y[mm]);
+        if (m == 0 && r.valid) r.y[(size_t)mm * r.ystride] = f2bf(tot);
+      }
+    }
+  }
+}
+
+// MFMA path, step 1: the operand (normalised when NORM) into the workspace's fragment
+// order. Workgroup = 16 rows x 256 values of a layer (K / 256 fastest, then row tiles); thread
+// (r, j) takes the 8 values 8 j of each of the two 128-value heads of row r, so a 16-lane DPP
+// row holds one head of one row and reads its contiguous bytes, and the head's sum of squares
+// is 8 terms per thread and a row sum. The 8 KB pass through LDS and leave in the workspace's
+// order, 256 bytes or more at a time. (One thread per 8 values storing its own 16 bytes, its
+// place found with 64-bit divisions, took 47-49 us for in_proj's 4096 rows, 14 us for 1024.)
+template <bool NORM>
+__global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p) {
+  __shared__ __attribute__((aligned(16))) u32x4 tile[512 + 512 / 16];  // 16 bytes of padding every 256
+  const int nch = p.K / 32, rows = 16 * p.mtiles;
+  const int npc = p.K / 256, piece = blockIdx.x % npc, mtl = blockIdx.x / npc;
+  const int mtile = mtl % p.mtiles, layer = mtl / p.mtiles;
+  const int r = threadIdx.x >> 4, j = threadIdx.x & 15;
+  const int mrow = 16 * mtile + r;
+  const bool live = mrow < p.M;
+  const size_t base = ((size_t)layer * p.M + (live ? mrow : 0)) * p.K + 256 * piece + 8 * j;
+  f4 gm[2];
+  NormIn in[2];
+  u16x8 x[2];
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh) {
+    if (NORM) in[hh] = norm_load(p, base + 128 * hh);
+    else x[hh] = *reinterpret_cast<const u16x8*>(p.x + base + 128 * hh);
+  }
+  if (NORM) {
+    const float* g = p.gamma + (size_t)layer * 128 + 8 * j;
+    gm[0] = *reinterpret_cast<const f4*>(g);
+    gm[1] = *reinterpret_cast<const f4*>(g + 4);
+  }
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh) {
+    float v[8];
+    if (NORM) {
+      gated_rmsnorm8(in[hh], gm, p.eps, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = live ? v[e] : 0.0f;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = live ? bf2f(x[hh][e]) : 0.0f;
+    }
+    u32x4 q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = pack_bf2(v[e], v[e + 4]);
+    // its place among the workgroup's 512 16-byte pieces: 32-value piece c of the 256, quarter
+    // jq of it
+    const int c = 4 * hh + (j >> 2), jq = j & 3;
+    const int at = p.frag32 ? (8 * (c >> 1) + 2 * jq + (c & 1)) * 16 + r
+                            : (2 * (c >> 1) + (jq & 1)) * 64 + 16 * (2 * (c & 1) + (jq >> 1)) + r;
+    tile[at + (at >> 4)] = q;
+    // the group's sum x: the 64 values of (row, group) are the 8 values of each of 8
+    // consecutive threads, added in a fixed order (each thread's 8 in sequence, then a
+    // butterfly over the 8 threads)
+    float sx = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sx += v[e];
+    sx += __shfl_xor(sx, 1, 8);
+    sx += __shfl_xor(sx, 2, 8);
+    sx += __shfl_xor(sx, 4, 8);
+    if ((j & 7) == 0)
+      p.xsum[((size_t)layer * (p.K / 64) + 4 * piece + 2 * hh + (j >> 3)) * rows + mrow] = sx;
+  }
+  __syncthreads();
+  u32x4* out = reinterpret_cast<u32x4*>(p.xfrag);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int at = 256 * i + threadIdx.x;
+    const u32x4 q = tile[at + (at >> 4)];
+    if (p.frag32) {
+      const int run = at >> 4;  // 16 rows of (group, block, half): 256 bytes
+      out[((size_t)layer * (p.mtiles / 2) + mtile / 2) * nch * 128 + (size_t)piece * 1024 + (run >> 1) * 64 +
+          (run & 1) * 32 + (mtile & 1) * 16 + (at & 15)] = q;
+    } else {
+      out[((size_t)layer * p.mtiles + mtile) * nch * 64 + (size_t)piece * 512 + at] = q;
+    }
+  }
+}
+
+__device__ __forceinline__ f4 mfma(bf8 a, bf8 b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// A nibble word (values k .. k + 7) as a B fragment: bf16 128 + v, pairs (i, i + 4).
+__device__ __forceinline__ bf8 nibbles_bf16(uint32_t wd, NibbleConsts k) {
+  u32x4 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = and_or(wd >> (4 * q), k.mask, k.bias);
+  return __builtin_bit_cast(bf8, r);
 }
 
 // MFMA path, step 2. Workgroup = 16 NT weight rows (the output columns) x 16 MT operand
@@ -1256,12 +1256,12 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
   }
 }
 
-template <bool NORM>
+template <bool NORM, int W, int NM>
 hipError_t launch_j(int J, const QParams& p, dim3 grid, size_t smem, hipStream_t stream) {
   switch (J) {
 #define GDN_QL_CASE(j) \
   case j:              \
-    hipLaunchKernelGGL((qlinear_kernel<j, NORM>), grid, dim3(kThreads), smem, stream, p); break;
+    hipLaunchKernelGGL((qlinear_kernel<j, NORM, W, NM>), grid, dim3(64 * W), smem, stream, p); break;
     GDN_QL_CASE(2) GDN_QL_CASE(4) GDN_QL_CASE(8) GDN_QL_CASE(10) GDN_QL_CASE(12) GDN_QL_CASE(16)
 #undef GDN_QL_CASE
     default:
@@ -1450,13 +1450,30 @@ hipError_t launch_qlinear(const gdn_qlinear_args& a, hipStream_t stream) {
   p.R = R;
   const bool norm = a.norm_x != nullptr;
   if (qlinear_uses_gemv(a.m, a.k)) {
-    // rows per workgroup: 64, or 256 with the norm prologue (every workgroup normalises
-    // the whole operand, so fewer, taller tiles)
-    p.passes = norm ? 16 : 4;
-    p.tiles = (R + kRowsPerPass * p.passes - 1) / (kRowsPerPass * p.passes);
+    // Waves and passes of 4 rows a wave per workgroup. One layer's rows in single passes put
+    // all of its weights in flight at once: in_proj at M = 1 16.3 us in 4 passes of 4 waves,
+    // 11.3 in one; M = 4 22.8 us in one pass of 8 waves, 24.5 of 4 waves (each wave reads the
+    // whole operand from LDS), 31.9 in 4 passes of 4. Calls of many rows fill the chip anyway
+    // and stage the operand less often in taller tiles (48 layers of in_proj at M = 4, per
+    // layer: 13.7 us in one pass, 12.1 in two; M = 1 6.7 with 1 to 4). With the norm every
+    // workgroup normalises the whole operand: the tallest tiles that still make 320
+    // workgroups, where one layer's 5120 rows take single passes (out_proj M = 1 9.0 us against
+    // 38 in 8 passes; 48 layers 2.8 us a layer in 8 passes, 3.2 in one).
+    const int W = norm || a.m > 2 ? 8 : 4;
+    const size_t rows = (size_t)a.n_layers * R;
+    if (norm) {
+      p.passes = 8;
+      while (p.passes > 1 && rows < (size_t)320 * 4 * W * p.passes) p.passes /= 2;
+    } else {
+      p.passes = rows < 131072 ? 1 : W == 8 ? 2 : 4;
+    }
+    p.tiles = (R + 4 * W * p.passes - 1) / (4 * W * p.passes);
     const dim3 grid((unsigned)((size_t)a.n_layers * p.tiles));
     const size_t smem = (size_t)p.M * (a.k / 32) * (4 * 16 + 4);
-    return norm ? launch_j<true>(a.k / 512, p, grid, smem, stream) : launch_j<false>(a.k / 512, p, grid, smem, stream);
+    const int J = a.k / 512;
+    if (norm) return a.m == 1 ? launch_j<true, 8, 1>(J, p, grid, smem, stream) : launch_j<true, 8, 4>(J, p, grid, smem, stream);
+    if (W == 8) return launch_j<false, 8, 4>(J, p, grid, smem, stream);
+    return a.m == 1 ? launch_j<false, 4, 1>(J, p, grid, smem, stream) : launch_j<false, 4, 4>(J, p, grid, smem, stream);
   }
   // MFMA path: the operand into the workspace, then the product
   const int MT = qgemm_mt(a.m);

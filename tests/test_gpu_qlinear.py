@@ -439,3 +439,37 @@ def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
         for l in range(L):
             check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], s[l][rows], b[l][rows]),
                   bound(O, x[l], s[l][rows], b[l][rows]), f"segment {i} layer {l}")
+
+
+# ---- GEMV tiles: one pass of 16 or 32 rows a workgroup, or several where the call has rows
+# enough (131,072 rows; with the norm 320 workgroups) ----
+
+@pytest.mark.parametrize("L,M,K,N,norm", [(8, 1, 1024, 16390, False), (8, 3, 1024, 16390, False),
+                                          (1, 2, 4096, 131100, False), (26, 1, 1024, 5121, True),
+                                          (3, 4, 2048, 7000, True)])
+def test_qlinear_gemv_passes(O, gdn, dev, L, M, K, N, norm):
+    import torch
+    log_case(f"qlinear (GEMV passes) L={L} M={M} K={K} N={N} norm={norm}")
+    rng = np.random.default_rng(L + M + N)
+    x, w, s, b = quant_inputs(O, L, M, N, K, seed=L + M + N)
+    sq = (lambda a: a) if L > 1 else (lambda a: a[0])
+    mat = dev_mat(gdn, dev, sq(w), sq(s), sq(b))
+    flip = np.zeros((L, M, 1))
+    if norm:
+        o = (rng.standard_normal((L, M, K)) * 0.3).astype(np.float32)
+        z = O.to_bf16(rng.standard_normal((L, M, K)).astype(np.float32))
+        gamma = rng.uniform(0.5, 1.5, (L, 128)).astype(np.float32)
+        (y,) = gdn.qlinear([mat], norm=(to_dev(sq(o), dev), to_dev(sq(z), dev), to_dev(sq(gamma), dev), 1e-6), n_layers=L)
+        x = np.stack([O.gated_rmsnorm(o[l].reshape(-1, 128), z[l].reshape(-1, 128), gamma[l], 1e-6).reshape(M, K)
+                      for l in range(L)])
+        flip = 3 * 2.0 ** -8 * np.abs(bf16_to_f32(x)).max(axis=2, keepdims=True)
+    else:
+        (y,) = gdn.qlinear([mat], to_dev(sq(x), dev), n_layers=L)
+    torch.cuda.synchronize()
+    got = to_np(y).reshape(L, M, N)
+    rows = sampled_rows(N, rng)
+    for l in range(L):
+        ss, bs = s[l][rows], b[l][rows]
+        wmax = (np.abs(bf16_to_f32(ss)) * 15 + np.abs(bf16_to_f32(bs))).max(axis=1)
+        check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], ss, bs),
+              bound(O, x[l], ss, bs) + flip[l] * wmax[None, :], f"layer {l}")
