@@ -16,7 +16,9 @@ library's message; nothing falls back to another implementation.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
+import struct
 from dataclasses import dataclass, field
 from typing import List, Optional
 
@@ -118,7 +120,30 @@ class QLinearArgs(ctypes.Structure):
     ]
 
 
+# The same structs for the calls that build their arguments themselves, packed from the fields
+# in order (null pointers as 0): filling a ctypes Structure takes 3-6 us of a call's host time,
+# packing its bytes about 1.
+_LAYER = struct.Struct("@6i3Pi4Pi9PiPiPNPi0P")
+_COMMIT = struct.Struct("@6iPi5PP")
+_QLINEAR = struct.Struct("@3i4Pfi" + "4Pi0P" * QLINEAR_MAX_SEGS + "PNP")
+for _s, _c in ((_LAYER, LayerArgs), (_COMMIT, CommitArgs), (_QLINEAR, QLinearArgs)):
+    if _s.size != ctypes.sizeof(_c):
+        raise ImportError(f"packed {_c.__name__} is {_s.size} bytes, the struct {ctypes.sizeof(_c)}")
+_NO_SEG = (0, 0, 0, 0, 0)
+
 _lib: Optional[ctypes.CDLL] = None
+_fast: dict = {}  # entry point name -> the function taking packed arguments
+
+
+def _call_packed(name: str, args: bytes) -> None:
+    f = _fast.get(name)
+    if f is None:
+        f = lib()[name]  # a function object of its own (attribute access shares one)
+        f.argtypes, f.restype = [ctypes.c_char_p], _int
+        _fast[name] = f
+    rc = f(args)
+    if rc != GDN_OK:
+        raise GdnError(rc, last_error())
 
 
 def lib() -> ctypes.CDLL:
@@ -196,6 +221,7 @@ def call_qlinear_noalloc(args: QLinearArgs) -> None:
     _check(lib().gdn_qlinear_noalloc(ctypes.byref(args)))
 
 
+@functools.lru_cache(maxsize=256)
 def qlinear_workspace_size(m: int, k: int, n_layers: int = 1) -> int:
     """Workspace bytes gdn_qlinear needs for m operand rows of k (0 on the GEMV path)."""
     a = QLinearArgs(n_layers=n_layers, m=m, k=k)
@@ -204,6 +230,7 @@ def qlinear_workspace_size(m: int, k: int, n_layers: int = 1) -> int:
     return n.value
 
 
+@functools.lru_cache(maxsize=256)
 def prefill_workspace_size(B: int, T: int, Hk: int = 16, Hv: int = 48, conv: bool = True,
                            precision: int = PREFILL_ACCURATE) -> int:
     """Workspace bytes of gdn_prefill_chunked; `conv` for the conv front end (x given),
@@ -219,8 +246,13 @@ def prefill_workspace_size(B: int, T: int, Hk: int = 16, Hv: int = 48, conv: boo
 # torch-facing helpers
 
 def _ptr(t) -> Optional[int]:
+    return None if t is None else _p(t)
+
+
+def _p(t) -> int:
+    """A tensor's address, 0 for None."""
     if t is None:
-        return None
+        return 0
     if not t.is_contiguous():
         raise GdnError(GDN_EINVAL, "tensors passed to libgdn must be contiguous")
     return t.data_ptr()
@@ -236,10 +268,23 @@ def _dt(t) -> int:
 
 
 def _stream(stream) -> Optional[int]:
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def _layer_call(name, *, B, T, Hk, Hv, q=None, k=None, v=None, x=None, conv_weight=None, conv_state_in=None,
+                conv_state_out=None, a=None, b=None, A_log=None, dt_bias=None, alpha=None, beta=None,
+                state_in=None, state_out=None, states=None, states_layout=STATES_BHT, o, workspace=None,
+                stream=None, precision=PREFILL_ACCURATE):
+    """gdn_run or gdn_prefill_chunked on one layer: layer_args's fields, packed."""
+    _call_packed(name, _LAYER.pack(
+        1, B, T, Hk, Hv, FRONTEND_QKV if x is None else FRONTEND_CONV, _p(q), _p(k), _p(v),
+        DTYPE_BF16 if q is None else _dt(q), _p(x), _p(conv_weight), _p(conv_state_in), _p(conv_state_out),
+        GATES_PRECOMPUTED if a is None else GATES_RAW, _p(a), _p(b), _p(A_log), _p(dt_bias), _p(alpha), _p(beta),
+        _p(state_in), _p(state_out), _p(states), states_layout, _p(o), _dt(o), _p(workspace),
+        0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream), precision))
 
 
 @dataclass
@@ -267,15 +312,10 @@ def run(q, k, v, alpha, beta, S=None, collect: bool = False, *, o_dtype=None, st
         s_out = torch.empty((B, H, HEAD_DIM, HEAD_DIM), dtype=torch.float32, device=q.device)
     S_all = (torch.empty((B, H, L, HEAD_DIM, HEAD_DIM), dtype=torch.float32, device=q.device)
              if collect else None)
-    args = LayerArgs(
-        n_layers=1, batch=B, seq_len=L, num_k_heads=q.shape[2], num_v_heads=v.shape[2],
-        frontend=FRONTEND_QKV, q=_ptr(q), k=_ptr(k), v=_ptr(v), qkv_dtype=_dt(q),
-        gate_mode=GATES_PRECOMPUTED, alpha=_ptr(alpha), beta=_ptr(beta),
-        state_in=_ptr(S), state_out=_ptr(s_out), states=_ptr(S_all), states_layout=STATES_BHT,
-        o=_ptr(o), o_dtype=_dt(o), stream=_stream(stream))
     if q.dtype != k.dtype or q.dtype != v.dtype:
         raise GdnError(GDN_EINVAL, "q, k, v must share a dtype")
-    call_run(args)
+    _layer_call("gdn_run", B=B, T=L, Hk=q.shape[2], Hv=v.shape[2], q=q, k=k, v=v, alpha=alpha, beta=beta,
+                state_in=S, state_out=s_out, states=S_all, o=o, stream=stream)
     states = [S_all[:, :, t] for t in range(L)] if collect else []
     return Result(o, s_out, states)
 
@@ -360,11 +400,10 @@ def layer(*, x=None, q=None, k=None, v=None, a, b, A_log, dt_bias, state=None,
         ws = workspace if workspace is not None else torch.empty(
             prefill_workspace_size(B, T, Hk, Hv, conv=x is not None, precision=precision), dtype=torch.uint8,
             device=dev)
-    args = layer_args(B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x, conv_weight=conv_weight,
-                      conv_state_in=conv_state, conv_state_out=conv_out, a=a, b=b,
-                      A_log=A_log, dt_bias=dt_bias, state_in=state, state_out=state_out,
-                      states=states, o=o, workspace=ws, stream=stream, precision=precision)
-    (call_prefill if chunked else call_run)(args)
+    _layer_call("gdn_prefill_chunked" if chunked else "gdn_run", B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x,
+                conv_weight=conv_weight, conv_state_in=conv_state, conv_state_out=conv_out, a=a, b=b,
+                A_log=A_log, dt_bias=dt_bias, state_in=state, state_out=state_out, states=states, o=o,
+                workspace=ws, stream=stream, precision=precision)
     return dict(o=o, state=state_out, states=states, conv_state=conv_out)
 
 
@@ -386,11 +425,10 @@ def prefill_chunked(*, x=None, q=None, k=None, v=None, a=None, b=None, A_log=Non
     if workspace is None and T > 0:
         workspace = torch.empty(prefill_workspace_size(B, T, Hk, Hv, conv=x is not None, precision=precision),
                                 dtype=torch.uint8, device=dev)
-    args = layer_args(B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x, conv_weight=conv_weight,
-                      conv_state_in=conv_state, conv_state_out=conv_out, a=a, b=b,
-                      A_log=A_log, dt_bias=dt_bias, alpha=alpha, beta=beta, state_in=state,
-                      state_out=state_out, o=o, workspace=workspace, stream=stream, precision=precision)
-    call_prefill(args)
+    _layer_call("gdn_prefill_chunked", B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x, conv_weight=conv_weight,
+                conv_state_in=conv_state, conv_state_out=conv_out, a=a, b=b, A_log=A_log, dt_bias=dt_bias,
+                alpha=alpha, beta=beta, state_in=state, state_out=state_out, o=o, workspace=workspace,
+                stream=stream, precision=precision)
     return dict(o=o, state=state_out, conv_state=conv_out)
 
 
@@ -400,12 +438,9 @@ def commit(*, n: int, T: int, states, state_prev, state_dst, x=None, conv_state_
     """DeltaCache::commit(n) on the device (cpp/src/model.cpp:439-457)."""
     B, Hv = state_dst.shape[-4], state_dst.shape[-3]
     C = x.shape[-1] if x is not None else (conv_state_dst.shape[-1] if conv_state_dst is not None else 0)
-    args = CommitArgs(n_layers=n_layers, batch=B, seq_len=T, num_v_heads=Hv, conv_dim=C, n=n,
-                      states=_ptr(states), states_layout=states_layout,
-                      state_prev=_ptr(state_prev), state_dst=_ptr(state_dst),
-                      conv_state_in=_ptr(conv_state_in), x=_ptr(x),
-                      conv_state_dst=_ptr(conv_state_dst), stream=_stream(stream))
-    call_commit(args)
+    _call_packed("gdn_commit", _COMMIT.pack(n_layers, B, T, Hv, C, n, _p(states), states_layout, _p(state_prev),
+                                            _p(state_dst), _p(conv_state_in), _p(x), _p(conv_state_dst),
+                                            _stream(stream)))
 
 
 class DeltaCache:
@@ -455,22 +490,18 @@ class DeltaCache:
         if self.record:
             states = torch.empty((T, B, self.Hv, HEAD_DIM, HEAD_DIM), dtype=torch.float32,
                                  device=x.device)
-            args = layer_args(B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x, conv_weight=conv_weight,
-                              conv_state_in=self.conv, a=a, b=b, A_log=A_log, dt_bias=dt_bias,
-                              state_in=self.state, states=states, states_layout=STATES_TBH,
-                              o=o, stream=stream)
-            call_run(args)
+            _layer_call("gdn_run", B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x, conv_weight=conv_weight,
+                        conv_state_in=self.conv, a=a, b=b, A_log=A_log, dt_bias=dt_bias, state_in=self.state,
+                        states=states, states_layout=STATES_TBH, o=o, stream=stream)
             self.base_offset = self.offset
             self.pending = (x, states, T)
         else:
             chunked = (self._ws is not None and T <= self.max_prefill_tokens
                        and _use_chunked(B, T, False, x, None, (x, o)))
-            args = layer_args(B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x, conv_weight=conv_weight,
-                              conv_state_in=self.conv, conv_state_out=self._conv_spare, a=a,
-                              b=b, A_log=A_log, dt_bias=dt_bias, state_in=self.state,
-                              state_out=self.state, o=o, workspace=self._ws if chunked else None,
-                              stream=stream, precision=self.prefill_precision)
-            (call_prefill if chunked else call_run)(args)
+            _layer_call("gdn_prefill_chunked" if chunked else "gdn_run", B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x,
+                        conv_weight=conv_weight, conv_state_in=self.conv, conv_state_out=self._conv_spare, a=a,
+                        b=b, A_log=A_log, dt_bias=dt_bias, state_in=self.state, state_out=self.state, o=o,
+                        workspace=self._ws if chunked else None, stream=stream, precision=self.prefill_precision)
             self.conv, self._conv_spare = self._conv_spare, self.conv
             self.offset += T
         return o
@@ -542,15 +573,45 @@ def qlinear_args(mats, x=None, *, norm=None, n_layers: int = 1, workspace=None, 
     return a, ys
 
 
+def _qlinear_call(name, mats, x, norm, n_layers, workspace, stream, alloc_workspace):
+    """qlinear_args's fields, packed, and the call; returns [y_i]."""
+    import torch
+    if len(mats) > QLINEAR_MAX_SEGS:
+        raise IndexError("invalid index")  # (as filling a gdn_qlinear_args does)
+    src = x if x is not None else norm[0]
+    M, K = src.shape[-2], src.shape[-1]
+    o = z = gamma = None
+    eps = 0.0
+    if norm is not None:
+        o, z, gamma, eps = norm
+    ys, segs = [], []
+    for q in mats:
+        n = q.w.shape[-2]
+        y = src.new_empty((n_layers, M, n) if n_layers > 1 else (M, n), dtype=torch.bfloat16)
+        ys.append(y)
+        segs += (_p(q.w), _p(q.scales), _p(q.biases), y.data_ptr(), n)
+    for _ in range(QLINEAR_MAX_SEGS - len(mats)):
+        segs += _NO_SEG
+    if workspace is None and alloc_workspace:
+        try:
+            need = qlinear_workspace_size(M, K, n_layers)
+        except GdnError:
+            need = 0  # a bad shape: gdn_qlinear itself reports it
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=src.device)
+    _call_packed(name, _QLINEAR.pack(
+        n_layers, M, K, _p(x), _p(o), _p(z), _p(gamma), eps, len(mats), *segs, _p(workspace),
+        0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream)))
+    return ys
+
+
 def qlinear(mats, x=None, *, norm=None, n_layers: int = 1, workspace=None, stream=None):
     """Linear::operator() for quantized weights (model.cpp:356-372) over 1..4 matrices
     sharing x -- e.g. the layer's in_proj_qkv, in_proj_z, in_proj_a, in_proj_b -- or, with
     norm = (o, z, gamma, eps), out_proj(GatedRMSNorm(o, z)) (model.cpp:626-641). Up to
     QLINEAR_GEMV_ROWS rows it is the GEMV kernel; more rows run on MFMA with a workspace
     (allocated here unless given)."""
-    args, ys = qlinear_args(mats, x, norm=norm, n_layers=n_layers, workspace=workspace, stream=stream)
-    call_qlinear(args)
-    return ys
+    return _qlinear_call("gdn_qlinear", mats, x, norm, n_layers, workspace, stream, True)
 
 
 def qlinear_noalloc(mats, x=None, *, norm=None, n_layers: int = 1, stream=None):
@@ -559,6 +620,4 @@ def qlinear_noalloc(mats, x=None, *, norm=None, n_layers: int = 1, stream=None):
     return GDN_EINVAL (e.g. M = 4096 at K = 5120 needs 41.25 MiB). Calls overlapping on one
     device race on the scratch. Only the outputs are allocated here; the library call itself
     allocates nothing."""
-    args, ys = qlinear_args(mats, x, norm=norm, n_layers=n_layers, stream=stream, alloc_workspace=False)
-    call_qlinear_noalloc(args)
-    return ys
+    return _qlinear_call("gdn_qlinear_noalloc", mats, x, norm, n_layers, None, stream, False)
