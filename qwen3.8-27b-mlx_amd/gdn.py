@@ -274,17 +274,21 @@ def _stream(stream) -> Optional[int]:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def _layer_call(name, *, B, T, Hk, Hv, q=None, k=None, v=None, x=None, conv_weight=None, conv_state_in=None,
+def _layer_call(chunked, *, B, T, Hk, Hv, q=None, k=None, v=None, x=None, conv_weight=None, conv_state_in=None,
                 conv_state_out=None, a=None, b=None, A_log=None, dt_bias=None, alpha=None, beta=None,
                 state_in=None, state_out=None, states=None, states_layout=STATES_BHT, o, workspace=None,
                 stream=None, precision=PREFILL_ACCURATE):
-    """gdn_run or gdn_prefill_chunked on one layer: layer_args's fields, packed."""
-    _call_packed(name, _LAYER.pack(
+    """gdn_run, or with `chunked` gdn_prefill_chunked, on one layer: layer_args's fields, packed."""
+    args = _LAYER.pack(
         1, B, T, Hk, Hv, FRONTEND_QKV if x is None else FRONTEND_CONV, _p(q), _p(k), _p(v),
         DTYPE_BF16 if q is None else _dt(q), _p(x), _p(conv_weight), _p(conv_state_in), _p(conv_state_out),
         GATES_PRECOMPUTED if a is None else GATES_RAW, _p(a), _p(b), _p(A_log), _p(dt_bias), _p(alpha), _p(beta),
         _p(state_in), _p(state_out), _p(states), states_layout, _p(o), _dt(o), _p(workspace),
-        0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream), precision))
+        0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream), precision)
+    if chunked:
+        call_prefill(LayerArgs.from_buffer_copy(args))  # (long enough for the structure's time not to matter)
+    else:
+        _call_packed("gdn_run", args)
 
 
 @dataclass
@@ -314,7 +318,7 @@ def run(q, k, v, alpha, beta, S=None, collect: bool = False, *, o_dtype=None, st
              if collect else None)
     if q.dtype != k.dtype or q.dtype != v.dtype:
         raise GdnError(GDN_EINVAL, "q, k, v must share a dtype")
-    _layer_call("gdn_run", B=B, T=L, Hk=q.shape[2], Hv=v.shape[2], q=q, k=k, v=v, alpha=alpha, beta=beta,
+    _layer_call(False, B=B, T=L, Hk=q.shape[2], Hv=v.shape[2], q=q, k=k, v=v, alpha=alpha, beta=beta,
                 state_in=S, state_out=s_out, states=S_all, o=o, stream=stream)
     states = [S_all[:, :, t] for t in range(L)] if collect else []
     return Result(o, s_out, states)
@@ -400,7 +404,7 @@ def layer(*, x=None, q=None, k=None, v=None, a, b, A_log, dt_bias, state=None,
         ws = workspace if workspace is not None else torch.empty(
             prefill_workspace_size(B, T, Hk, Hv, conv=x is not None, precision=precision), dtype=torch.uint8,
             device=dev)
-    _layer_call("gdn_prefill_chunked" if chunked else "gdn_run", B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x,
+    _layer_call(chunked, B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x,
                 conv_weight=conv_weight, conv_state_in=conv_state, conv_state_out=conv_out, a=a, b=b,
                 A_log=A_log, dt_bias=dt_bias, state_in=state, state_out=state_out, states=states, o=o,
                 workspace=ws, stream=stream, precision=precision)
@@ -425,7 +429,7 @@ def prefill_chunked(*, x=None, q=None, k=None, v=None, a=None, b=None, A_log=Non
     if workspace is None and T > 0:
         workspace = torch.empty(prefill_workspace_size(B, T, Hk, Hv, conv=x is not None, precision=precision),
                                 dtype=torch.uint8, device=dev)
-    _layer_call("gdn_prefill_chunked", B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x, conv_weight=conv_weight,
+    _layer_call(True, B=B, T=T, Hk=Hk, Hv=Hv, q=q, k=k, v=v, x=x, conv_weight=conv_weight,
                 conv_state_in=conv_state, conv_state_out=conv_out, a=a, b=b, A_log=A_log, dt_bias=dt_bias,
                 alpha=alpha, beta=beta, state_in=state, state_out=state_out, o=o, workspace=workspace,
                 stream=stream, precision=precision)
@@ -490,7 +494,7 @@ class DeltaCache:
         if self.record:
             states = torch.empty((T, B, self.Hv, HEAD_DIM, HEAD_DIM), dtype=torch.float32,
                                  device=x.device)
-            _layer_call("gdn_run", B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x, conv_weight=conv_weight,
+            _layer_call(False, B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x, conv_weight=conv_weight,
                         conv_state_in=self.conv, a=a, b=b, A_log=A_log, dt_bias=dt_bias, state_in=self.state,
                         states=states, states_layout=STATES_TBH, o=o, stream=stream)
             self.base_offset = self.offset
@@ -498,7 +502,7 @@ class DeltaCache:
         else:
             chunked = (self._ws is not None and T <= self.max_prefill_tokens
                        and _use_chunked(B, T, False, x, None, (x, o)))
-            _layer_call("gdn_prefill_chunked" if chunked else "gdn_run", B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x,
+            _layer_call(chunked, B=B, T=T, Hk=self.Hk, Hv=self.Hv, x=x,
                         conv_weight=conv_weight, conv_state_in=self.conv, conv_state_out=self._conv_spare, a=a,
                         b=b, A_log=A_log, dt_bias=dt_bias, state_in=self.state, state_out=self.state, o=o,
                         workspace=self._ws if chunked else None, stream=stream, precision=self.prefill_precision)
