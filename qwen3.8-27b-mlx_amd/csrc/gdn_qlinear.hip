@@ -79,7 +79,8 @@ struct QParams {
   // values k = 64 g + 32 h + 8 s + (0, 4, 1, 5, 2, 6, 3, 7)
   int frag32;
   int mgroups;  // MFMA path: groups of MT m-tiles (the grid is layers x tiles x mgroups)
-  int remap;    // MFMA path: XCD-aware workgroup order (see qgemm_kernel)
+  int remap;    // MFMA path: XCD-aware workgroup order (see qgemm_tile)
+  int layers;   // qgemm_big_kernel's leftover rows
 };
 
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
@@ -444,27 +445,30 @@ __device__ __forceinline__ bf8 nibbles_bf16(uint32_t wd, NibbleConsts k) {
 constexpr int kRing = 2;  // groups in flight per wave (G / 4 is a multiple of it)
 // F32: the operand is in qgemm_big_kernel's 32-row fragments (its leftover rows): this lane's
 // values are block 2 (g4 % 2) + s of group g there, lane 32 (g4 / 2) + 16 (mt % 2) + nn.
-template <int MT, int NT, bool F32>
-__global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
-  constexpr int kRows = 16 * NT;
-  constexpr int kMaxG = 8192 / 64;
+template <int MT, int NT>
+struct QgemmLds {
+  static constexpr int kRows = 16 * NT;
+  static constexpr int kMaxG = 8192 / 64;
   // scale | bias << 16 per (row, group), rows kMaxG + 1 words apart at most (a row stride
   // of G + 1 words puts the 16 rows a wave reads at once on distinct banks); at the end the
   // partial sums of waves 1..3
-  __shared__ __attribute__((aligned(16))) union {
+  union {
     uint32_t sb[kRows * (kMaxG + 1)];
     f4 red[3][MT * NT][64];
-  } sm;
+  };
   // the operand's group sums for this workgroup's MT m tiles, all groups: [group][16 MT]
-  __shared__ __attribute__((aligned(16))) float xs_l[kMaxG * 16 * MT];
+  __attribute__((aligned(16))) float xs_l[kMaxG * 16 * MT];
+};
+template <int MT, int NT, bool F32>
+__device__ __forceinline__ void qgemm_tile(const QParams& p, int bid, int nwg, QgemmLds<MT, NT>& sm) {
+  constexpr int kRows = 16 * NT;
   // Workgroup = (layer, weight tile, m group), m groups fastest. Workgroups are dispatched to
   // the 8 XCDs round robin; the ids are renumbered (p.remap) so that each XCD runs a
   // contiguous range: with several m groups, all m groups of a weight tile on one XCD, one
   // after another, so its weight rows come from HBM once and from that XCD's L2 after; with
   // 8 layers or more, whole layers per XCD, so a layer's operand is read from HBM into one
   // L2 instead of all eight.
-  int bid = blockIdx.x;
-  if (p.remap) bid = (bid & 7) * (int)(gridDim.x >> 3) + (bid >> 3);
+  if (p.remap) bid = (bid & 7) * (nwg >> 3) + (bid >> 3);
   const int mg = bid % p.mgroups, lt = bid / p.mgroups;
   const int layer = lt / p.tiles, tile = lt % p.tiles;
   const int mt0 = mg * MT;
@@ -544,7 +548,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
     const float* xsg = p.xsum + (size_t)layer * G * (16 * p.mtiles) + 16 * mt0;
     for (int q = threadIdx.x; q < 4 * MT * G; q += kThreads) {
       const int g = q / (4 * MT), o = 4 * (q % (4 * MT));
-      *reinterpret_cast<f4*>(&xs_l[g * 16 * MT + o]) = *reinterpret_cast<const f4*>(xsg + (size_t)g * 16 * p.mtiles + o);
+      *reinterpret_cast<f4*>(&sm.xs_l[g * 16 * MT + o]) = *reinterpret_cast<const f4*>(xsg + (size_t)g * 16 * p.mtiles + o);
     }
   }
   __syncthreads();
@@ -560,7 +564,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
     const int g = 4 * i + wave;
     f4 xs[MT];  // sum x of the group for this lane's rows 4 g4 .. + 3 of each m tile
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xs[mt] = *reinterpret_cast<const f4*>(&xs_l[g * 16 * MT + 16 * mt + 4 * g4]);
+    for (int mt = 0; mt < MT; ++mt) xs[mt] = *reinterpret_cast<const f4*>(&sm.xs_l[g * 16 * MT + 16 * mt + 4 * g4]);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const uint32_t sbv = sm.sb[(16 * nt + nn) * sbs + g];
@@ -610,6 +614,12 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
         }
       }
   }
+}
+
+template <int MT, int NT>
+__global__ __launch_bounds__(kThreads) void qgemm_kernel(QParams p) {
+  __shared__ __attribute__((aligned(16))) QgemmLds<MT, NT> sm;
+  qgemm_tile<MT, NT, false>(p, blockIdx.x, gridDim.x, sm);
 }
 
 // MFMA path for calls of many weight rows and few operand rows (one m group of up to 48 rows;
@@ -934,6 +944,7 @@ __device__ __forceinline__ bf8 nibbles16_bf16(uint32_t wd, NibbleConsts k) {
   return __builtin_bit_cast(bf8, r);
 }
 constexpr int kBigSlots = 3;
+constexpr int kRestTiles = 2;  // 16-row tiles of a workgroup of leftover rows
 template <int WN, int WK, int MTW>
 struct BigCfg {
   static constexpr int NTW = 2;                    // 32-row weight tiles of a wave
@@ -947,8 +958,12 @@ struct BigCfg {
   static_assert(WN * WK == 4 && MTW * WK == 4, "4 waves share each step's loads evenly");
 };
 
-template <int WN, int WK, int MTW>
-__global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
+// The rows past each matrix's whole tiles (r: in_proj_a and in_proj_b are all such rows) are
+// qgemm_kernel's tiles, in the first `nrest` workgroups of the same launch: in a launch of
+// their own the in_proj's 96 rows took 17 us after 1024 operand rows and 40 us after 4096, here
+// they run beside the first tiles.
+template <int WN, int WK, int MTW, bool REST>
+__global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p, QParams r, int nrest) {
   using C = BigCfg<WN, WK, MTW>;
   constexpr int NTW = C::NTW;
   __shared__ __attribute__((aligned(16))) unsigned char smem[C::kLds];
@@ -958,7 +973,14 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p) {
   // tile ids, in which panels of 8 weight tiles run weight tile fastest, so the tiles one XCD
   // runs at once share their weight and operand slices through its L2.
   int bid = blockIdx.x;
-  if (p.remap) bid = (bid & 7) * (int)(gridDim.x >> 3) + (bid >> 3);
+  if (REST && bid < nrest) {
+    static_assert(sizeof(QgemmLds<4, kRestTiles>) <= C::kLds, "the leftover rows' tiles fit the same LDS");
+    if (bid < r.tiles * r.mgroups * r.layers)
+      qgemm_tile<4, kRestTiles, true>(r, bid, 0, *reinterpret_cast<QgemmLds<4, kRestTiles>*>(smem));
+    return;
+  }
+  if (REST) bid -= nrest;  // (a multiple of 8: the XCDs keep their turns)
+  if (p.remap) bid = (bid & 7) * (int)((gridDim.x - (REST ? nrest : 0)) >> 3) + (bid >> 3);
   const int per_layer = p.tiles * p.mgroups;
   const int layer = bid / per_layer;
   int rem = bid % per_layer;
@@ -1289,35 +1311,14 @@ int qgemm_mtiles(int m) {
   return ((m + 15) / 16 + mt - 1) / mt * mt;
 }
 
-template <int MT, bool F32>
+template <int MT>
 hipError_t launch_gemm_mt(int NT, const QParams& p, dim3 grid, hipStream_t stream) {
   switch (NT) {
-    case 1: hipLaunchKernelGGL((qgemm_kernel<MT, 1, F32>), grid, dim3(kThreads), 0, stream, p); break;
-    case 2: hipLaunchKernelGGL((qgemm_kernel<MT, 2, F32>), grid, dim3(kThreads), 0, stream, p); break;
-    default: hipLaunchKernelGGL((qgemm_kernel<MT, 4, F32>), grid, dim3(kThreads), 0, stream, p); break;
+    case 1: hipLaunchKernelGGL((qgemm_kernel<MT, 1>), grid, dim3(kThreads), 0, stream, p); break;
+    case 2: hipLaunchKernelGGL((qgemm_kernel<MT, 2>), grid, dim3(kThreads), 0, stream, p); break;
+    default: hipLaunchKernelGGL((qgemm_kernel<MT, 4>), grid, dim3(kThreads), 0, stream, p); break;
   }
   return hipGetLastError();
-}
-
-// qgemm_kernel over the p.R rows of p: MT m tiles and NT row tiles per workgroup
-template <bool F32>
-hipError_t launch_gemm(QParams p, int n_layers, int MT, hipStream_t stream) {
-  const int gy = p.mtiles / MT;
-  // weight rows per workgroup: 64, 32 or 16 -- the most that still gives 512 workgroups
-  int NT = 4;
-  while (NT > 1 && (size_t)n_layers * ((p.R + 16 * NT - 1) / (16 * NT)) * gy < 512) NT /= 2;
-  p.tiles = (p.R + 16 * NT - 1) / (16 * NT);
-  p.mgroups = gy;
-  const size_t nwg = (size_t)n_layers * p.tiles * gy;
-  p.remap = (gy > 1 || n_layers >= 8) && nwg % 8 == 0;
-  const dim3 grid((unsigned)nwg);
-  if (F32) return launch_gemm_mt<4, F32>(NT, p, grid, stream);  // (its operand has whole 64-row groups)
-  switch (MT) {
-    case 1: return launch_gemm_mt<1, false>(NT, p, grid, stream);
-    case 2: return launch_gemm_mt<2, false>(NT, p, grid, stream);
-    case 3: return launch_gemm_mt<3, false>(NT, p, grid, stream);
-    default: return launch_gemm_mt<4, false>(NT, p, grid, stream);
-  }
 }
 
 // The weight rows qgemm_big_kernel takes of an n-row matrix, in whole tiles of `rows`; a last
@@ -1335,15 +1336,15 @@ size_t big_workgroups(const QParams& p, int n_layers, int per_cu) {
 // Which form of the product a call of more than 48 rows takes: 0 qgemm_kernel, 1 the 128 x 256
 // tiles, 2 the 64 x 128 ones (K split in two). Measured at K = 5120 and 6144 (the layer's
 // projections), a CU with n workgroups takes about 85 n + 10 us with the large tiles and
-// 24 n + 24 us with the small ones: in_proj M = 333 109 (large) / 101 us, M = 512 117 / 125,
-// M = 1024 190 / 223, M = 4096 700 / 871; out_proj M = 1024 117 / 107, M = 2048 197 / 181,
-// M = 4096 342 / 349. With few small tiles most CUs stand idle and qgemm_kernel's 64 x 64 tiles
-// split over more workgroups are faster: out_proj M = 128 (80 tiles) 37 us against 45, in_proj
-// M = 64 (128) 47 against 52; from 160 (out_proj M = 256) 47 against 56, in_proj M = 128 (256)
-// 55 against 62.
+// 24 n + 24 us with the small ones: in_proj M = 512 117 (large) / 125 us, M = 1024 190 / 223,
+// M = 4096 700 / 871; out_proj M = 1024 117 / 107, M = 2048 197 / 181, M = 4096 342 / 349. With
+// few small tiles most CUs stand idle and qgemm_kernel's 64 x 64 tiles split over more
+// workgroups are faster: out_proj M = 128 (80 tiles) 37 us against 45; from 120 on the small
+// tiles are as fast or faster (out_proj M = 160 to 192, 120 tiles: 45 us both; in_proj M = 64,
+// 128 tiles: 38 against 45).
 int big_form(const QParams& p, int n_layers) {
   constexpr int kCUs = 256;
-  if (big_workgroups<2, 2, 2>(p, n_layers, 1) < 144) return 0;
+  if (big_workgroups<2, 2, 2>(p, n_layers, 1) < 100) return 0;
   const size_t large = big_workgroups<4, 1, 4>(p, n_layers, kCUs), small = big_workgroups<2, 2, 2>(p, n_layers, kCUs);
   return big_workgroups<4, 1, 4>(p, n_layers, 1) > 0 && 85 * large + 10 <= 24 * small + 24 ? 1 : 2;
 }
@@ -1360,11 +1361,7 @@ hipError_t launch_big(QParams p, int n_layers, hipStream_t stream) {
   p.mgroups = (p.mtiles / 2 + MTW - 1) / MTW;
   const size_t nwg = (size_t)n_layers * p.tiles * p.mgroups;
   p.remap = nwg % 8 == 0;
-  hipLaunchKernelGGL((qgemm_big_kernel<WN, WK, MTW>), dim3((unsigned)nwg), dim3(kThreads), 0, stream, p);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  // the rows past the whole tiles (in_proj_a and in_proj_b are all such rows)
-  QParams r = p;
+  QParams r = p;  // the rows past the whole tiles
   r.nseg = 0;
   r.R = 0;
   for (int q = 0; q < p.nseg; ++q) {
@@ -1379,7 +1376,15 @@ hipError_t launch_big(QParams p, int n_layers, hipStream_t stream) {
     r.row0[i] = r.R;
     r.R += p.n[q] - done;
   }
-  return r.R ? launch_gemm<true>(r, n_layers, 4, stream) : hipSuccess;
+  r.layers = n_layers;
+  r.tiles = (r.R + 16 * kRestTiles - 1) / (16 * kRestTiles);
+  r.mgroups = p.mtiles / 4;
+  r.remap = 0;
+  const size_t nrest = ((size_t)n_layers * r.tiles * r.mgroups + 7) / 8 * 8;
+  const dim3 grid((unsigned)(nrest + nwg));
+  if (nrest) hipLaunchKernelGGL((qgemm_big_kernel<WN, WK, MTW, true>), grid, dim3(kThreads), 0, stream, p, r, (int)nrest);
+  else hipLaunchKernelGGL((qgemm_big_kernel<WN, WK, MTW, false>), grid, dim3(kThreads), 0, stream, p, r, 0);
+  return hipGetLastError();
 }
 }  // namespace
 
@@ -1513,7 +1518,21 @@ hipError_t launch_qlinear(const gdn_qlinear_args& a, hipStream_t stream) {
     }
     return hipGetLastError();
   }
-  return launch_gemm<false>(p, a.n_layers, MT, stream);
+  // weight rows per workgroup: 64, 32 or 16 -- the most that still gives 512 workgroups
+  const int gy = p.mtiles / MT;
+  int NT = 4;
+  while (NT > 1 && (size_t)a.n_layers * ((R + 16 * NT - 1) / (16 * NT)) * gy < 512) NT /= 2;
+  p.tiles = (R + 16 * NT - 1) / (16 * NT);
+  p.mgroups = gy;
+  const size_t nwg = (size_t)a.n_layers * p.tiles * gy;
+  p.remap = (gy > 1 || a.n_layers >= 8) && nwg % 8 == 0;
+  const dim3 grid((unsigned)nwg);
+  switch (MT) {
+    case 1: return launch_gemm_mt<1>(NT, p, grid, stream);
+    case 2: return launch_gemm_mt<2>(NT, p, grid, stream);
+    case 3: return launch_gemm_mt<3>(NT, p, grid, stream);
+    default: return launch_gemm_mt<4>(NT, p, grid, stream);
+  }
 }
 
 }  // namespace gdn

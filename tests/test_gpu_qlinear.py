@@ -409,12 +409,14 @@ def test_qlinear_4096_rows_two_layers(O, gdn, dev):
 
 
 # ---- the LDS-tiled product (qgemm_big_kernel) ----
-# Calls of more than 48 rows and at least 144 tiles of 64 operand x 128 weight rows take it, in
+# Calls of more than 48 rows and at least 100 tiles of 64 operand x 128 weight rows take it, in
 # tiles of 64 x 128 or (few enough workgroups a CU, see big_form) 128 x 256. A matrix's rows past
-# its whole tiles are a partial tile where it is 5/8 full, else qgemm_kernel's.
+# its whole tiles are a partial tile where it is 5/8 full, else qgemm_kernel's tiles in the same
+# launch.
 
 @pytest.mark.parametrize("L,M,K,ns", [
     (1, 129, 1024, [6200, 100, 48]),   # 64 x 128: 48 tiles + 56 rows, a partial tile, a matrix of leftovers only
+    (1, 49, 1024, [12800 + 33]),       # the fewest rows and tiles: 100, and 33 leftover rows
     (2, 65, 2048, [5000]),             # two layers, one operand row in the second 64
     (1, 260, 8192, [4096 + 7]),        # the longest K, seven leftover rows
     (1, 1000, 1024, [8000, 200, 24]),  # 128 x 256: 31 tiles + 64 rows, a partial tile, leftovers only
