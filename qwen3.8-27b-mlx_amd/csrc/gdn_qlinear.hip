@@ -1334,19 +1334,20 @@ size_t big_workgroups(const QParams& p, int n_layers, int per_cu) {
 }
 
 // Which form of the product a call of more than 48 rows takes: 0 qgemm_kernel, 1 the 128 x 256
-// tiles, 2 the 64 x 128 ones (K split in two). Measured at K = 5120 and 6144 (the layer's
-// projections), a CU with n workgroups takes about 85 n + 10 us with the large tiles and
-// 24 n + 24 us with the small ones: in_proj M = 512 117 (large) / 125 us, M = 1024 190 / 223,
-// M = 4096 700 / 871; out_proj M = 1024 117 / 107, M = 2048 197 / 181, M = 4096 342 / 349. With
-// few small tiles most CUs stand idle and qgemm_kernel's 64 x 64 tiles split over more
-// workgroups are faster: out_proj M = 128 (80 tiles) 37 us against 45; from 120 on the small
-// tiles are as fast or faster (out_proj M = 160 to 192, 120 tiles: 45 us both; in_proj M = 64,
-// 128 tiles: 38 against 45).
+// tiles, 2 the 64 x 128 ones (K split in two). Measured at K = 5120 (and 6/5 of it at 6144), a
+// CU with n workgroups takes about 85 n + 8 us with the large tiles and 27.5 n us with the small
+// ones; large / small tiles over rotated operands: in_proj M = 333 105 / 101 us, M = 512 114 /
+// 124, M = 700 162 / 165, M = 1024 194 / 240; out_proj M = 512 122 / 68, M = 1024 133 / 111,
+// M = 1536 141 / 147, M = 2048 200 / 187, M = 4096 346 / 376 (qgemm_kernel at M = 512 and 1024
+// 75 and 126). With few small tiles most CUs stand idle and qgemm_kernel's 64 x 64 tiles split
+// over more workgroups are faster: out_proj M = 128 (80 tiles) 37 us against 45; from 120 on
+// the small tiles are as fast or faster (out_proj M = 160 to 192, 120 tiles: 45 us both; in_proj
+// M = 64, 128 tiles: 38 against 45).
 int big_form(const QParams& p, int n_layers) {
   constexpr int kCUs = 256;
   if (big_workgroups<2, 2, 2>(p, n_layers, 1) < 100) return 0;
   const size_t large = big_workgroups<4, 1, 4>(p, n_layers, kCUs), small = big_workgroups<2, 2, 2>(p, n_layers, kCUs);
-  return big_workgroups<4, 1, 4>(p, n_layers, 1) > 0 && 85 * large + 10 <= 24 * small + 24 ? 1 : 2;
+  return big_workgroups<4, 1, 4>(p, n_layers, 1) > 0 && 170 * large + 16 <= 55 * small ? 1 : 2;
 }
 
 template <int WN, int WK, int MTW>

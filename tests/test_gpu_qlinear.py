@@ -420,7 +420,7 @@ def test_qlinear_4096_rows_two_layers(O, gdn, dev):
     (2, 65, 2048, [5000]),             # two layers, one operand row in the second 64
     (1, 260, 8192, [4096 + 7]),        # the longest K, seven leftover rows
     (1, 1000, 1024, [8000, 200, 24]),  # 128 x 256: 31 tiles + 64 rows, a partial tile, leftovers only
-    (1, 897, 5120, [8192 + 255]),      # a partial tile of 255 rows; one row in the last 128
+    (1, 897, 5120, [7936 + 255]),      # 128 x 256: a partial tile of 255 rows; one row in the last 128
 ])
 def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
     import torch
