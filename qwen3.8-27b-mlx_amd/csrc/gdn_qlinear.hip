@@ -18,7 +18,7 @@
 // bias are applied once per half-group: sum x (q s + b) = s * sum x (128 + q) +
 // (b - 128 s) * sum x. The row total is a DPP row sum; the result is rounded to bf16 once.
 //
-// More rows (verify blocks, batched decode) run on MFMA (v_mfma_f32_16x16x32_bf16) with the
+// More rows (verify blocks, batched decode, prefill windows) run on MFMA with the
 // same arithmetic: qprep writes the operand once into the workspace in the MFMA fragment
 // order (the norm prologue applied there, as above) together with each row's sum x per
 // 64-value group, then in qgemm each lane's weight row gives B fragments straight from its
@@ -27,7 +27,8 @@
 // workgroup's 4 waves split K and add their partial sums in LDS at the end, so each wave
 // reads a quarter of the operand; calls of many weight rows and one m group (up to 64 rows,
 // e.g. 8 layers of in_proj at once) take qgemm_ns instead, whose workgroup of 256 weight rows
-// reads the operand into LDS once for its four waves.
+// reads the operand into LDS once for its four waves; calls of more than 48 rows and enough
+// tiles take qgemm_big, whose workgroups share 128 x 256 or 64 x 128 tiles through LDS.
 #include "../../include/gdn.h"
 #include "gdn_device_math.h"
 #include "gdn_internal.h"
