@@ -234,29 +234,7 @@ __global__ __launch_bounds__(64 * W) void qlinear_kernel(QParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int passes = p.passes;
 
-  // a pass's rows: the lane's row and the words it loads of it -- the scale and bias words, 16
-  // bytes a lane (groups 8 mc .. + 7; lanes past the row's K / 512 chunks repeat the last),
-  // first: they arrive before the weights
-  struct Row {
-    uint16_t* y;
-    int ystride;
-    bool valid;
-    u32x4 s, b, w[J];
-  };
-  const int mc = m < J ? m : J - 1;
-  auto load = [&](int pass, Row& r) {
-    const int grow = (tile * passes + pass) * (4 * W) + wave * 4 + (lane >> 4);
-    r.valid = grow < p.R;
-    const int row = r.valid ? grow : p.R - 1;
-    const RowPtrs rp = row_ptrs(p, layer, row);
-    g_u32x4* wr = (g_u32x4*)rp.w;
-    r.s = *(g_u32x4*)(rp.s + 8 * mc);
-    r.b = *(g_u32x4*)(rp.b + 8 * mc);
-#pragma unroll
-    for (int j = 0; j < J; ++j) r.w[j] = __builtin_nontemporal_load(wr + m + 16 * j);
-    r.y = rp.y;
-    r.ystride = rp.ystride;
-  };
+  const int mc = m < J ? m : J - 1;  // the 8 groups whose scale and bias words the lane loads
 
   // ---- stage the operand ----
   if (NORM) {
@@ -296,14 +274,49 @@ __global__ __launch_bounds__(64 * W) void qlinear_kernel(QParams p) {
   // ---- passes of 4 rows per wave ----
   const NibbleConsts nk = nibble_consts();
   for (int pass = 0; pass < passes; ++pass) {
-    Row r;
-    load(pass, r);
+    // (the operand is read from LDS again in every pass: without branches between the products
+    // the compiler would hold all of it in registers, 253 at K = 5120)
+    if (NM == 1) asm volatile("" ::: "memory");
+    const int grow = (tile * passes + pass) * (4 * W) + wave * 4 + (lane >> 4);
+    const bool valid = grow < p.R;
+    const int row = valid ? grow : p.R - 1;
+    // the row's segment, selected here in the kernel's body: through row_ptrs the selection held
+    // more registers than there are scalar ones and took about 85 vector instructions a pass more,
+    // with K a variable (M = 2, 48 layers of in_proj 384-393 us against 376; K = 1024, 248,320
+    // rows 38 us against 33)
+    int sg = 0;
+#pragma unroll
+    for (int q = 1; q < GDN_QLINEAR_MAX_SEGS; ++q) sg += (q < p.nseg && row >= p.row0[q]) ? 1 : 0;
+    const uint32_t* wseg = p.w[0];
+    const uint16_t *sseg = p.s[0], *bseg = p.b[0];
+    uint16_t* yseg = p.y[0];
+    int nseg = p.n[0], r0 = p.row0[0];
+#pragma unroll
+    for (int q = 1; q < GDN_QLINEAR_MAX_SEGS; ++q) {
+      if (sg == q) {
+        wseg = p.w[q];
+        sseg = p.s[q];
+        bseg = p.b[q];
+        yseg = p.y[q];
+        nseg = p.n[q];
+        r0 = p.row0[q];
+      }
+    }
+    // the row's scale and bias words, 16 bytes a lane (groups 8 mc .. + 7; lanes past the row's
+    // K / 512 chunks repeat the last), first: they arrive before the weights
+    const size_t lrow = (size_t)layer * nseg + (row - r0);
+    const u32x4* wr = reinterpret_cast<const u32x4*>(wseg + lrow * (K / 8));
+    const u32x4 swd = *reinterpret_cast<const u32x4*>(sseg + lrow * (K / 64) + 8 * mc);
+    const u32x4 bwd = *reinterpret_cast<const u32x4*>(bseg + lrow * (K / 64) + 8 * mc);
+    u32x4 wv[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) wv[j] = __builtin_nontemporal_load(wr + m + 16 * j);
     // through this wave's LDS rows (written and read by this wave only: no barrier) to the
     // lanes that use them: piece m + 16 j is in group m / 2 + 8 j
     uint16_t* srl = &sbs[wave][lane >> 4][0][0];
     uint16_t* brl = &sbs[wave][lane >> 4][1][0];
-    *reinterpret_cast<u32x4*>(srl + 8 * mc) = r.s;
-    *reinterpret_cast<u32x4*>(brl + 8 * mc) = r.b;
+    *reinterpret_cast<u32x4*>(srl + 8 * mc) = swd;
+    *reinterpret_cast<u32x4*>(brl + 8 * mc) = bwd;
     float y[NM] = {};
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -313,7 +326,7 @@ __global__ __launch_bounds__(64 * W) void qlinear_kernel(QParams p) {
       uint32_t pr[4][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint32_t wd = r.w[j][i];
+        const uint32_t wd = wv[j][i];
 #pragma unroll
         for (int q = 0; q < 4; ++q) pr[i][q] = and_or(wd >> (4 * q), nk.mask, nk.bias);
       }
@@ -335,7 +348,7 @@ __global__ __launch_bounds__(64 * W) void qlinear_kernel(QParams p) {
     for (int mm = 0; mm < NM; ++mm) {
       if (NM == 1 || mm < p.M) {
         const float tot = row16_sum(y[mm]);
-        if (m == 0 && r.valid) r.y[(size_t)mm * r.ystride] = f2bf(tot);
+        if (m == 0 && valid) yseg[((size_t)layer * p.M + mm) * nseg + (row - r0)] = f2bf(tot);
       }
     }
   }

@@ -475,3 +475,23 @@ def test_qlinear_gemv_passes(O, gdn, dev, L, M, K, N, norm):
         wmax = (np.abs(bf16_to_f32(ss)) * 15 + np.abs(bf16_to_f32(bs))).max(axis=1)
         check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], ss, bs),
               bound(O, x[l], ss, bs) + flip[l] * wmax[None, :], f"layer {l}")
+
+
+@pytest.mark.parametrize("M", [1, 2, 4])
+def test_qlinear_gemv_segment_bounds(O, gdn, dev, M):
+    """Four matrices whose bounds fall inside the four rows a wave takes, two layers."""
+    import torch
+    log_case(f"qlinear (GEMV) segments of 33, 2, 18, 5 rows x 2 layers, M={M}, K=2048")
+    L, K = 2, 2048
+    mats, host, x = [], [], None
+    for i, n in enumerate([33, 2, 18, 5]):
+        xi, w, s, b = quant_inputs(O, L, M, n, K, seed=1700 + 10 * M + i)
+        x = xi if x is None else x
+        mats.append(dev_mat(gdn, dev, w, s, b))
+        host.append((w, s, b))
+    ys = gdn.qlinear(mats, to_dev(x, dev), n_layers=L)
+    torch.cuda.synchronize()
+    for i, ((w, s, b), y) in enumerate(zip(host, ys)):
+        got = to_np(y)
+        for l in range(L):
+            check(got[l], O.qlinear(x[l], w[l], s[l], b[l]), bound(O, x[l], s[l], b[l]), f"segment {i} layer {l}")
