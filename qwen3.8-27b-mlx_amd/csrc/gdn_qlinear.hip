@@ -1470,22 +1470,35 @@ hipError_t launch_qlinear(const gdn_qlinear_args& a, hipStream_t stream) {
   p.R = R;
   const bool norm = a.norm_x != nullptr;
   if (qlinear_uses_gemv(a.m, a.k)) {
-    // Waves and passes of 4 rows a wave per workgroup. One layer's rows in single passes put
-    // all of its weights in flight at once: in_proj at M = 1 16.3 us in 4 passes of 4 waves,
-    // 11.3 in one; M = 4 22.8 us in one pass of 8 waves, 24.5 of 4 waves (each wave reads the
-    // whole operand from LDS), 31.9 in 4 passes of 4. Calls of many rows fill the chip anyway
-    // and stage the operand less often in taller tiles (48 layers of in_proj at M = 4, per
-    // layer: 13.7 us in one pass, 12.1 in two; M = 1 6.7 with 1 to 4). With the norm every
-    // workgroup normalises the whole operand: the tallest tiles that still make 320
-    // workgroups, where one layer's 5120 rows take single passes (out_proj M = 1 9.0 us against
-    // 38 in 8 passes; 48 layers 2.8 us a layer in 8 passes, 3.2 in one).
-    const int W = norm || a.m > 2 ? 8 : 4;
+    // Waves and passes of 4 rows a wave per workgroup. Calls of few rows take single passes, which
+    // put all of their weights in flight at once: in_proj at M = 1 10.7 us in one pass of 4 waves,
+    // 15.8 in four; M = 4 21.6 us in one pass of 8 waves, 22.8 of 4 waves (each wave reads the
+    // whole operand from LDS), 30 in four passes of 4. Calls of many rows fill the chip anyway and
+    // stage the operand less often in taller tiles. At K = 5120: M = 1 one pass of 4 waves up to
+    // 7 layers of in_proj (115,360 rows; 51.2 us, in four 57), then two (24 layers 162, in four
+    // 166; at K = 8192 four: 140,000 rows 98.4, in two 100.9); M = 2 one pass up to 5 (82,400
+    // rows; 47.0, in two 47.5), then two (7 layers 63.8; in one 66.4, in four 64.8), from 131,072
+    // rows four (48 layers 376; in two 392); M = 3 and 4 8 waves in one pass up to 5 layers (M = 4
+    // 68.9, in two 69.2), then two (7 layers 90.3, in one 92.2), but in one to 131,072 rows where
+    // the operand's LDS leaves a CU few workgroups (M = 4, K = 6144, 120,000 rows: 108 against
+    // 112). At K = 1024 a pass is short against the staging: from 65,536 rows 4 waves and several
+    // passes (69,632 rows: M = 1 10.1 us in four, 11.0 in one; M = 4 15.6 in two, 16.8 in one of 8
+    // waves; 248,320 rows: M = 4 45.2 in four, 46.3 in two of 8 waves).
+    // With the norm every workgroup normalises the whole operand: the tallest tiles that still make
+    // 320 workgroups, where one layer's 5120 rows take single passes (out_proj M = 1 9.0 us
+    // against 38 in 8 passes; 48 layers 2.8 us a layer in 8 passes, 3.2 in one).
     const size_t rows = (size_t)a.n_layers * R;
+    const bool shortk = a.k == 1024 && rows >= 65536;
+    const int W = norm || (a.m > 2 && !shortk) ? 8 : 4;
     if (norm) {
       p.passes = 8;
       while (p.passes > 1 && rows < (size_t)320 * 4 * W * p.passes) p.passes /= 2;
+    } else if (W == 8) {
+      p.passes = rows < (a.m * a.k > 20480 ? 131072 : 98304) ? 1 : 2;
+    } else if (a.m == 1) {
+      p.passes = rows < 131072 && !shortk ? 1 : a.k > 1024 && a.k < 8192 ? 2 : 4;
     } else {
-      p.passes = rows < 131072 ? 1 : W == 8 ? 2 : 4;
+      p.passes = rows < 98304 && !shortk ? 1 : rows < 131072 ? 2 : 4;
     }
     p.tiles = (R + 4 * W * p.passes - 1) / (4 * W * p.passes);
     const dim3 grid((unsigned)((size_t)a.n_layers * p.tiles));

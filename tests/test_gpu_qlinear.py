@@ -444,11 +444,12 @@ def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
 
 
 # ---- GEMV tiles: one pass of 16 or 32 rows a workgroup, or several where the call has rows
-# enough (131,072 rows; with the norm 320 workgroups) ----
+# enough (65,536 rows at K = 1024, else 98,304 or 131,072; with the norm 320 workgroups) ----
 
 @pytest.mark.parametrize("L,M,K,N,norm", [(8, 1, 1024, 16390, False), (8, 3, 1024, 16390, False),
                                           (1, 2, 4096, 131100, False), (26, 1, 1024, 5121, True),
-                                          (3, 4, 2048, 7000, True)])
+                                          (3, 4, 2048, 7000, True), (1, 2, 2048, 98310, False),
+                                          (1, 3, 2048, 98330, False), (1, 4, 1024, 65570, False)])
 def test_qlinear_gemv_passes(O, gdn, dev, L, M, K, N, norm):
     import torch
     log_case(f"qlinear (GEMV passes) L={L} M={M} K={K} N={N} norm={norm}")
