@@ -355,27 +355,27 @@ __global__ __launch_bounds__(64 * W) void qlinear_kernel(QParams p) {
 }
 
 // MFMA path, step 1: the operand (normalised when NORM) into the workspace's fragment
-// order. Workgroup = 16 rows x 256 values of a layer (K / 256 fastest, then row tiles); thread
-// (r, j) takes the 8 values 8 j of each of the two 128-value heads of row r, so a 16-lane DPP
-// row holds one head of one row and reads its contiguous bytes, and the head's sum of squares
-// is 8 terms per thread and a row sum. The 8 KB pass through LDS and leave in the workspace's
+// order. Workgroup = 16 rows x 128 HH values of a layer (K / (128 HH) fastest, then row tiles);
+// thread (r, j) takes the 8 values 8 j of each of the HH 128-value heads of row r, so a 16-lane
+// DPP row holds one head of one row and reads its contiguous bytes, and the head's sum of squares
+// is 8 terms per thread and a row sum. The 4 HH KB pass through LDS and leave in the workspace's
 // order, 256 bytes or more at a time. (One thread per 8 values storing its own 16 bytes, its
 // place found with 64-bit divisions, took 47-49 us for in_proj's 4096 rows, 14 us for 1024.)
-template <bool NORM>
+template <bool NORM, int HH>
 __global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p) {
-  __shared__ __attribute__((aligned(16))) u32x4 tile[512 + 512 / 16];  // 16 bytes of padding every 256
+  __shared__ __attribute__((aligned(16))) u32x4 tile[HH * (256 + 256 / 16)];  // 16 bytes of padding every 256
   const int nch = p.K / 32, rows = 16 * p.mtiles;
-  const int npc = p.K / 256, piece = blockIdx.x % npc, mtl = blockIdx.x / npc;
+  const int npc = p.K / (128 * HH), piece = blockIdx.x % npc, mtl = blockIdx.x / npc;
   const int mtile = mtl % p.mtiles, layer = mtl / p.mtiles;
   const int r = threadIdx.x >> 4, j = threadIdx.x & 15;
   const int mrow = 16 * mtile + r;
   const bool live = mrow < p.M;
-  const size_t base = ((size_t)layer * p.M + (live ? mrow : 0)) * p.K + 256 * piece + 8 * j;
+  const size_t base = ((size_t)layer * p.M + (live ? mrow : 0)) * p.K + 128 * HH * piece + 8 * j;
   f4 gm[2];
-  NormIn in[2];
-  u16x8 x[2];
+  NormIn in[HH];
+  u16x8 x[HH];
 #pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
+  for (int hh = 0; hh < HH; ++hh) {
     if (NORM) in[hh] = norm_load(p, base + 128 * hh);
     else x[hh] = *reinterpret_cast<const u16x8*>(p.x + base + 128 * hh);
   }
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p) {
     gm[1] = *reinterpret_cast<const f4*>(g + 4);
   }
 #pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
+  for (int hh = 0; hh < HH; ++hh) {
     float v[8];
     if (NORM) {
       gated_rmsnorm8(in[hh], gm, p.eps, v);
@@ -398,8 +398,8 @@ __global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p) {
     u32x4 q;
 #pragma unroll
     for (int e = 0; e < 4; ++e) q[e] = pack_bf2(v[e], v[e + 4]);
-    // its place among the workgroup's 512 16-byte pieces: 32-value piece c of the 256, quarter
-    // jq of it
+    // its place among the workgroup's 256 HH 16-byte pieces: 32-value piece c of its values,
+    // quarter jq of it
     const int c = 4 * hh + (j >> 2), jq = j & 3;
     const int at = p.frag32 ? (8 * (c >> 1) + 2 * jq + (c & 1)) * 16 + r
                             : (2 * (c >> 1) + (jq & 1)) * 64 + 16 * (2 * (c & 1) + (jq >> 1)) + r;
@@ -414,20 +414,20 @@ __global__ __launch_bounds__(kThreads) void qprep_kernel(QParams p) {
     sx += __shfl_xor(sx, 2, 8);
     sx += __shfl_xor(sx, 4, 8);
     if ((j & 7) == 0)
-      p.xsum[((size_t)layer * (p.K / 64) + 4 * piece + 2 * hh + (j >> 3)) * rows + mrow] = sx;
+      p.xsum[((size_t)layer * (p.K / 64) + 2 * HH * piece + 2 * hh + (j >> 3)) * rows + mrow] = sx;
   }
   __syncthreads();
   u32x4* out = reinterpret_cast<u32x4*>(p.xfrag);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < HH; ++i) {
     const int at = 256 * i + threadIdx.x;
     const u32x4 q = tile[at + (at >> 4)];
     if (p.frag32) {
       const int run = at >> 4;  // 16 rows of (group, block, half): 256 bytes
-      out[((size_t)layer * (p.mtiles / 2) + mtile / 2) * nch * 128 + (size_t)piece * 1024 + (run >> 1) * 64 +
+      out[((size_t)layer * (p.mtiles / 2) + mtile / 2) * nch * 128 + (size_t)piece * (512 * HH) + (run >> 1) * 64 +
           (run & 1) * 32 + (mtile & 1) * 16 + (at & 15)] = q;
     } else {
-      out[((size_t)layer * p.mtiles + mtile) * nch * 64 + (size_t)piece * 512 + at] = q;
+      out[((size_t)layer * p.mtiles + mtile) * nch * 64 + (size_t)piece * (256 * HH) + at] = q;
     }
   }
 }
@@ -1523,9 +1523,19 @@ hipError_t launch_qlinear(const gdn_qlinear_args& a, hipStream_t stream) {
   }
   const int big = sb16 && off32 && p.mtiles > 3 ? big_form(p, a.n_layers) : 0;
   p.frag32 = big != 0;
-  const dim3 gp((unsigned)((size_t)a.n_layers * p.mtiles * (a.k / 256)));
-  if (norm) hipLaunchKernelGGL(qprep_kernel<true>, gp, dim3(kThreads), 0, stream, p);
-  else hipLaunchKernelGGL(qprep_kernel<false>, gp, dim3(kThreads), 0, stream, p);
+  // One head a thread: with two, the calls of few rows had half the workgroups and each did two
+  // norms in sequence (out_proj M = 5 13.9 us against 13.1, M = 333 47.6 against 45.7); from 4096
+  // workgroups of two they are enough (out_proj M = 4096 333 us against 336).
+  const size_t np = (size_t)a.n_layers * p.mtiles * (a.k / 256);
+  if (np < 4096) {
+    const dim3 gp((unsigned)(2 * np));
+    if (norm) hipLaunchKernelGGL((qprep_kernel<true, 1>), gp, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((qprep_kernel<false, 1>), gp, dim3(kThreads), 0, stream, p);
+  } else {
+    const dim3 gp((unsigned)np);
+    if (norm) hipLaunchKernelGGL((qprep_kernel<true, 2>), gp, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((qprep_kernel<false, 2>), gp, dim3(kThreads), 0, stream, p);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (big == 1) return launch_big<4, 1, 4>(p, a.n_layers, stream);

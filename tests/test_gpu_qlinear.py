@@ -496,3 +496,28 @@ def test_qlinear_gemv_segment_bounds(O, gdn, dev, M):
         got = to_np(y)
         for l in range(L):
             check(got[l], O.qlinear(x[l], w[l], s[l], b[l]), bound(O, x[l], s[l], b[l]), f"segment {i} layer {l}")
+
+
+# ---- the operand's preparation: one head a thread, or from 4096 workgroups two ----
+
+@pytest.mark.parametrize("M,N", [(4096, 40), (4096, 384), (1984, 40)])  # two heads, both layouts; one head
+@pytest.mark.parametrize("norm", [False, True])
+def test_qlinear_operand_preparation(O, gdn, dev, M, N, norm):
+    import torch
+    log_case(f"qlinear (operand preparation) M={M} N={N} K=8192 norm={norm}")
+    K = 8192
+    rng = np.random.default_rng(M + N)
+    x, w, s, b = quant_inputs(O, 1, M, N, K, seed=M + N)
+    mat, x, flip = dev_mat(gdn, dev, w[0], s[0], b[0]), x[0], 0.0
+    if norm:
+        o = (rng.standard_normal((M, K)) * 0.3).astype(np.float32)
+        z = O.to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+        gamma = rng.uniform(0.5, 1.5, 128).astype(np.float32)
+        (y,) = gdn.qlinear([mat], norm=(to_dev(o, dev), to_dev(z, dev), to_dev(gamma, dev), 1e-6))
+        x = O.gated_rmsnorm(o.reshape(-1, 128), z.reshape(-1, 128), gamma, 1e-6).reshape(M, K)
+        wmax = (np.abs(bf16_to_f32(s[0])) * 15 + np.abs(bf16_to_f32(b[0]))).max(axis=1)
+        flip = 3 * 2.0 ** -8 * np.abs(bf16_to_f32(x)).max(axis=1, keepdims=True) * wmax[None, :]
+    else:
+        (y,) = gdn.qlinear([mat], to_dev(x, dev))
+    torch.cuda.synchronize()
+    check(to_np(y), O.qlinear_blocked(x, w[0], s[0], b[0]), bound(O, x, s[0], b[0]) + flip, "y")
