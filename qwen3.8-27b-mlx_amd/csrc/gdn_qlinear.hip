@@ -1356,10 +1356,14 @@ size_t big_workgroups(const QParams& p, int n_layers, int per_cu) {
 // 75 and 126). With few small tiles most CUs stand idle and qgemm_kernel's 64 x 64 tiles split
 // over more workgroups are faster: out_proj M = 128 (80 tiles) 37 us against 45; from 120 on
 // the small tiles are as fast or faster (out_proj M = 160 to 192, 120 tiles: 45 us both; in_proj
-// M = 64, 128 tiles: 38 against 45).
+// M = 64, 128 tiles: 38 against 45). But where qgemm_kernel's 64 x 32 tiles are exactly two
+// workgroups a CU it is faster up to 16 m groups: at N = 4096, M = 256 the 128 small tiles take
+// 36.2 us for K = 5120 and 52.7 for K = 8192, qgemm_kernel 28.6 and 40.4; N = 16384, M = 64,
+// K = 5120 39.5 and 36.0; N = 1024, M = 1024 39.3 and 33.3; N = 512, M = 2048 42.2 and 47.9.
 int big_form(const QParams& p, int n_layers) {
   constexpr int kCUs = 256;
   if (big_workgroups<2, 2, 2>(p, n_layers, 1) < 100) return 0;
+  if (p.mtiles / 4 <= 16 && (size_t)n_layers * ((p.R + 31) / 32) * (p.mtiles / 4) == 2 * kCUs) return 0;
   const size_t large = big_workgroups<4, 1, 4>(p, n_layers, kCUs), small = big_workgroups<2, 2, 2>(p, n_layers, kCUs);
   return big_workgroups<4, 1, 4>(p, n_layers, 1) > 0 && 170 * large + 16 <= 55 * small ? 1 : 2;
 }

@@ -443,6 +443,24 @@ def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
                   bound(O, x[l], s[l][rows], b[l][rows]), f"segment {i} layer {l}")
 
 
+# ---- qgemm_kernel's 64 x 32 tiles where they are exactly two workgroups a CU (512): big_form ----
+
+@pytest.mark.parametrize("L,M,N,K", [(1, 256, 4096, 1024), (1, 50, 16370, 1024), (2, 100, 4090, 2048)])
+def test_qlinear_mfma_512_workgroups(O, gdn, dev, L, M, N, K):
+    import torch
+    log_case(f"qlinear (MFMA path, 512 workgroups) L={L} M={M} N={N} K={K}")
+    rng = np.random.default_rng(M + N)
+    x, w, s, b = quant_inputs(O, L, M, N, K, seed=M + N)
+    sq = (lambda a: a) if L > 1 else (lambda a: a[0])
+    (y,) = gdn.qlinear([dev_mat(gdn, dev, sq(w), sq(s), sq(b))], to_dev(sq(x), dev), n_layers=L)
+    torch.cuda.synchronize()
+    got = to_np(y).reshape(L, M, N)
+    rows = sampled_rows(N, rng)
+    for l in range(L):
+        check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], s[l][rows], b[l][rows]),
+              bound(O, x[l], s[l][rows], b[l][rows]), f"layer {l}")
+
+
 # ---- GEMV tiles: one pass of 16 or 32 rows a workgroup, or several where the call has rows
 # enough (65,536 rows at K = 1024, else 98,304 or 131,072; with the norm 320 workgroups) ----
 
