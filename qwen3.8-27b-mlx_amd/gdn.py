@@ -590,7 +590,7 @@ def _qlinear_call(name, mats, x, norm, n_layers, workspace, stream, alloc_worksp
         o, z, gamma, eps = norm
     ys, segs = [], []
     for q in mats:
-        n = q.w.shape[-2]
+        n = q.n
         y = src.new_empty((n_layers, M, n) if n_layers > 1 else (M, n), dtype=torch.bfloat16)
         ys.append(y)
         segs += (_p(q.w), _p(q.scales), _p(q.biases), y.data_ptr(), n)

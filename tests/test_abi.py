@@ -7,6 +7,7 @@ import ctypes
 import os
 import re
 import subprocess
+import types
 
 import pytest
 
@@ -363,3 +364,38 @@ def test_length_dispatch_follows_the_measured_crossover(gdn):
         assert not use(B, first - 1, False, x, None, (x,))
         assert use(B, first, False, x, None, (x,))
         assert not use(B, 4096, True, x, None, (x,))
+
+
+# ---- the packed argument structs of the calls that build their own ----
+
+STREAM = types.SimpleNamespace(cuda_stream=0x77700)
+
+
+@pytest.fixture
+def packed(gdn, monkeypatch):
+    """What the calls hand to the library, as (entry point, bytes); nothing is called."""
+    calls = []
+    monkeypatch.setattr(gdn.gdn, "_call_packed", lambda name, args: calls.append((name, bytes(args))))
+    return calls
+
+
+def _mats(gdn, sizes, K=1024, cls=None):
+    import torch
+    return [(cls or gdn.QuantLinear)(torch.zeros((n, K // 8), dtype=torch.int32),
+                                     torch.zeros((n, K // 64), dtype=torch.bfloat16),
+                                     torch.zeros((n, K // 64), dtype=torch.bfloat16)) for n in sizes]
+
+
+def test_qlinear_takes_the_rows_the_weight_states(gdn, packed):
+    """The output's width and the call's rows are the weight's `n`, as in qlinear_args."""
+    import torch
+
+    class Rows(gdn.QuantLinear):
+        @property
+        def n(self):
+            return self.w.shape[-2] - 3
+
+    x = torch.zeros((2, 1024), dtype=torch.bfloat16)
+    (y,) = gdn.qlinear(_mats(gdn, [40], cls=Rows), x, stream=STREAM)
+    a = gdn.QLinearArgs.from_buffer_copy(packed[0][1])
+    assert y.shape == (2, 37) and a.segs[0].n == 37
