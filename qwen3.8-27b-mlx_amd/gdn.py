@@ -221,7 +221,7 @@ def call_qlinear_noalloc(args: QLinearArgs) -> None:
     _check(lib().gdn_qlinear_noalloc(ctypes.byref(args)))
 
 
-@functools.lru_cache(maxsize=256)
+@functools.lru_cache(maxsize=256, typed=True)
 def qlinear_workspace_size(m: int, k: int, n_layers: int = 1) -> int:
     """Workspace bytes gdn_qlinear needs for m operand rows of k (0 on the GEMV path)."""
     a = QLinearArgs(n_layers=n_layers, m=m, k=k)
@@ -230,7 +230,7 @@ def qlinear_workspace_size(m: int, k: int, n_layers: int = 1) -> int:
     return n.value
 
 
-@functools.lru_cache(maxsize=256)
+@functools.lru_cache(maxsize=256, typed=True)
 def prefill_workspace_size(B: int, T: int, Hk: int = 16, Hv: int = 48, conv: bool = True,
                            precision: int = PREFILL_ACCURATE) -> int:
     """Workspace bytes of gdn_prefill_chunked; `conv` for the conv front end (x given),

@@ -399,3 +399,11 @@ def test_qlinear_takes_the_rows_the_weight_states(gdn, packed):
     (y,) = gdn.qlinear(_mats(gdn, [40], cls=Rows), x, stream=STREAM)
     a = gdn.QLinearArgs.from_buffer_copy(packed[0][1])
     assert y.shape == (2, 37) and a.segs[0].n == 37
+
+
+def test_workspace_sizes_take_whole_numbers_only(gdn):
+    """A size kept for (40, 5120) answers no call for (40.0, 5120)."""
+    for f, whole in ((gdn.qlinear_workspace_size, (40, 5120)), (gdn.prefill_workspace_size, (1, 100))):
+        f(*whole)
+        with pytest.raises(TypeError):
+            f(float(whole[0]), whole[1])
