@@ -131,6 +131,29 @@ for _s, _c in ((_LAYER, LayerArgs), (_COMMIT, CommitArgs), (_QLINEAR, QLinearArg
         raise ImportError(f"packed {_c.__name__} is {_s.size} bytes, the struct {ctypes.sizeof(_c)}")
 _NO_SEG = (0, 0, 0, 0, 0)
 
+
+def _fill(cls, values):
+    """A `cls` from its fields' values in order, as ctypes converts or refuses them."""
+    a = cls()
+    for name, ct in cls._fields_:
+        if issubclass(ct, ctypes.Array):
+            for i in range(ct._length_):
+                getattr(a, name)[i] = _fill(ct._type_, values)
+        else:
+            setattr(a, name, next(values))
+    return a
+
+
+def _pack(fmt: struct.Struct, cls, *values) -> bytes:
+    """The bytes of a `cls`. What struct refuses -- other types, numbers out of a field's range --
+    ctypes decides."""
+    try:
+        return fmt.pack(*values)
+    except (struct.error, OverflowError):
+        return bytes(_fill(cls, iter(values)))
+
+
+
 _lib: Optional[ctypes.CDLL] = None
 _fast: dict = {}  # entry point name -> the function taking packed arguments
 
@@ -279,8 +302,8 @@ def _layer_call(chunked, *, B, T, Hk, Hv, q=None, k=None, v=None, x=None, conv_w
                 state_in=None, state_out=None, states=None, states_layout=STATES_BHT, o, workspace=None,
                 stream=None, precision=PREFILL_ACCURATE):
     """gdn_run, or with `chunked` gdn_prefill_chunked, on one layer: layer_args's fields, packed."""
-    args = _LAYER.pack(
-        1, B, T, Hk, Hv, FRONTEND_QKV if x is None else FRONTEND_CONV, _p(q), _p(k), _p(v),
+    args = _pack(
+        _LAYER, LayerArgs, 1, B, T, Hk, Hv, FRONTEND_QKV if x is None else FRONTEND_CONV, _p(q), _p(k), _p(v),
         DTYPE_BF16 if q is None else _dt(q), _p(x), _p(conv_weight), _p(conv_state_in), _p(conv_state_out),
         GATES_PRECOMPUTED if a is None else GATES_RAW, _p(a), _p(b), _p(A_log), _p(dt_bias), _p(alpha), _p(beta),
         _p(state_in), _p(state_out), _p(states), states_layout, _p(o), _dt(o), _p(workspace),
@@ -442,9 +465,9 @@ def commit(*, n: int, T: int, states, state_prev, state_dst, x=None, conv_state_
     """DeltaCache::commit(n) on the device (cpp/src/model.cpp:439-457)."""
     B, Hv = state_dst.shape[-4], state_dst.shape[-3]
     C = x.shape[-1] if x is not None else (conv_state_dst.shape[-1] if conv_state_dst is not None else 0)
-    _call_packed("gdn_commit", _COMMIT.pack(n_layers, B, T, Hv, C, n, _p(states), states_layout, _p(state_prev),
-                                            _p(state_dst), _p(conv_state_in), _p(x), _p(conv_state_dst),
-                                            _stream(stream)))
+    _call_packed("gdn_commit", _pack(_COMMIT, CommitArgs, n_layers, B, T, Hv, C, n, _p(states), states_layout,
+                                     _p(state_prev), _p(state_dst), _p(conv_state_in), _p(x), _p(conv_state_dst),
+                                     _stream(stream)))
 
 
 class DeltaCache:
@@ -588,6 +611,7 @@ def _qlinear_call(name, mats, x, norm, n_layers, workspace, stream, alloc_worksp
     eps = 0.0
     if norm is not None:
         o, z, gamma, eps = norm
+        eps = float(eps)
     ys, segs = [], []
     for q in mats:
         n = q.n
@@ -603,8 +627,8 @@ def _qlinear_call(name, mats, x, norm, n_layers, workspace, stream, alloc_worksp
             need = 0  # a bad shape: gdn_qlinear itself reports it
         if need:
             workspace = torch.empty(need, dtype=torch.uint8, device=src.device)
-    _call_packed(name, _QLINEAR.pack(
-        n_layers, M, K, _p(x), _p(o), _p(z), _p(gamma), eps, len(mats), *segs, _p(workspace),
+    _call_packed(name, _pack(
+        _QLINEAR, QLinearArgs, n_layers, M, K, _p(x), _p(o), _p(z), _p(gamma), eps, len(mats), *segs, _p(workspace),
         0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream)))
     return ys
 

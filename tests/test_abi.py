@@ -407,3 +407,30 @@ def test_workspace_sizes_take_whole_numbers_only(gdn):
         f(*whole)
         with pytest.raises(TypeError):
             f(float(whole[0]), whole[1])
+
+
+@pytest.mark.parametrize("n", [2 ** 31, -2 ** 31 - 1, 2 ** 32 + 1])
+def test_packed_arguments_wrap_as_the_struct_does(gdn, packed, n):
+    """A count past 32 bits reaches the library as the struct converts it, which judges it."""
+    import torch
+    state = torch.zeros((1, 48, 128, 128))
+    gdn.commit(n=n, T=4, states=None, state_prev=state, state_dst=state, stream=STREAM)
+    got = gdn.CommitArgs.from_buffer_copy(packed[0][1])
+    assert got.n == gdn.CommitArgs(n=n).n and got.seq_len == 4 and got.stream == STREAM.cuda_stream
+    assert got.state_prev == got.state_dst == state.data_ptr()
+
+
+def test_packed_arguments_refuse_what_the_struct_refuses(gdn, packed):
+    import torch
+    state = torch.zeros((1, 48, 128, 128))
+    with pytest.raises(TypeError):
+        gdn.commit(n=1.0, T=4, states=None, state_prev=state, state_dst=state, stream=STREAM)
+    o, z, gamma = torch.zeros((2, 1024)), torch.zeros((2, 1024), dtype=torch.bfloat16), torch.ones(128)
+    with pytest.raises(TypeError):
+        gdn.qlinear(_mats(gdn, [8]), norm=(o, z, gamma, None), stream=STREAM)
+    assert not packed
+    for eps, want in (("1e-6", 1e-6), (1e39, float("inf")), (torch.tensor(0.5), 0.5)):
+        gdn.qlinear(_mats(gdn, [8, 9]), norm=(o, z, gamma, eps), stream=STREAM)
+        a = gdn.QLinearArgs.from_buffer_copy(packed.pop()[1])
+        assert a.norm_eps == ctypes.c_float(want).value
+        assert (a.n_segs, a.segs[0].n, a.segs[1].n, a.segs[2].n, a.stream) == (2, 8, 9, 0, STREAM.cuda_stream)
