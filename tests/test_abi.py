@@ -434,3 +434,11 @@ def test_packed_arguments_refuse_what_the_struct_refuses(gdn, packed):
         a = gdn.QLinearArgs.from_buffer_copy(packed.pop()[1])
         assert a.norm_eps == ctypes.c_float(want).value
         assert (a.n_segs, a.segs[0].n, a.segs[1].n, a.segs[2].n, a.stream) == (2, 8, 9, 0, STREAM.cuda_stream)
+
+
+def test_current_stream_without_the_raw_accessor(gdn, monkeypatch):
+    """Where torch has no raw accessor for the current stream, the public one gives it."""
+    import torch
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: STREAM)
+    assert gdn.gdn._stream(None) == STREAM.cuda_stream
