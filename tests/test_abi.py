@@ -442,3 +442,55 @@ def test_current_stream_without_the_raw_accessor(gdn, monkeypatch):
     monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: STREAM)
     assert gdn.gdn._stream(None) == STREAM.cuda_stream
+
+
+def _distinct(names, **dtypes):
+    """One small tensor a name, each with its own address."""
+    import torch
+    return {k: torch.zeros(64, dtype=getattr(torch, dtypes.get(k, "float32"))) for k in names.split()}
+
+
+@pytest.mark.parametrize("chunked", [False, True])
+@pytest.mark.parametrize("conv", [False, True])
+@pytest.mark.parametrize("raw", [False, True])
+def test_packed_layer_fields_are_layer_args_fields(gdn, packed, monkeypatch, chunked, conv, raw):
+    """Every field of a packed call at its place: the bytes of the struct layer_args fills."""
+    sent = []
+    monkeypatch.setattr(gdn.gdn, "call_prefill", lambda a: sent.append(bytes(a)))
+    names = "q k v conv_weight conv_state_in conv_state_out b A_log dt_bias alpha beta state_in state_out states o workspace"
+    t = _distinct(names + " x" * conv + " a" * raw, o="bfloat16", workspace="uint8")
+    kw = dict(t, B=3, T=5, Hk=8, Hv=24, states_layout=gdn.STATES_TBH, stream=STREAM, precision=gdn.PREFILL_FAST)
+    gdn.gdn._layer_call(chunked, **kw)
+    (got,) = sent if chunked else [args for name, args in packed if name == "gdn_run"]
+    assert got == bytes(gdn.layer_args(**kw))
+
+
+def test_packed_commit_fields_are_the_structs(gdn, packed):
+    import torch
+    t = _distinct("states state_prev conv_state_in x conv_state_dst", x="bfloat16")
+    t["state_dst"] = torch.zeros((2, 3, 1, 1))
+    gdn.commit(n=4, T=5, n_layers=6, states_layout=gdn.STATES_TBH, stream=STREAM, **t)
+    want = gdn.CommitArgs(n_layers=6, batch=2, seq_len=5, num_v_heads=3, conv_dim=64, n=4,
+                          states_layout=gdn.STATES_TBH, stream=STREAM.cuda_stream,
+                          **{k: v.data_ptr() for k, v in t.items()})
+    assert packed == [("gdn_commit", bytes(want))]
+
+
+@pytest.mark.parametrize("sizes", [[8], [8, 9, 10, 11]])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_packed_qlinear_fields_are_qlinear_args_fields(gdn, packed, sizes, norm, noalloc):
+    import torch
+    mats = _mats(gdn, sizes)
+    rows = (torch.zeros((40, 1024)), torch.zeros((40, 1024), dtype=torch.bfloat16), torch.ones(128), 1e-5)
+    kw = dict(norm=rows) if norm else dict(x=rows[1])
+    if noalloc:
+        ys = gdn.qlinear_noalloc(mats, stream=STREAM, **kw)
+        want, _ = gdn.qlinear_args(mats, stream=STREAM, alloc_workspace=False, **kw)
+    else:
+        ws = torch.empty(gdn.qlinear_workspace_size(40, 1024), dtype=torch.uint8)
+        ys = gdn.qlinear(mats, workspace=ws, stream=STREAM, **kw)
+        want, _ = gdn.qlinear_args(mats, workspace=ws, stream=STREAM, **kw)
+    for i, y in enumerate(ys):  # each call makes its own outputs
+        want.segs[i].y = y.data_ptr()
+    assert packed == [("gdn_qlinear_noalloc" if noalloc else "gdn_qlinear", bytes(want))]

@@ -3,8 +3,8 @@
 626-641) -- against the oracle's fp64 dequantize-and-dot.
 
 Tolerance: the result is rounded to bf16 once (half an ulp: at most 2^-8 relative), and the fp32
-accumulation (products of x with the offset bf16 values 128 + nibble, per 32-value piece)
-adds at most 2^-20 of sum_k |x_k| (143 |s_k| + |b_k|), the magnitudes it accumulates. The
+accumulation (products of x with the offset bf16 values 128 + nibble, per 32-value piece;
+16 + nibble in the LDS-tiled form) adds at most 2^-20 of sum_k |x_k| (143 |s_k| + |b_k|), the magnitudes it accumulates. The
 test allows 2^-8 |y| plus that bound. MLX's own accumulation order is unpinned at bit
 level; the reference rounds its fp32 result to bf16 as this does.
 """
@@ -200,14 +200,16 @@ def test_qlinear_mfma_reuses_a_caller_workspace(O, gdn, dev):
         check(to_np(y), O.qlinear(x[0], w[0], s[0], b[0]), bound(O, x[0], s[0], b[0]), f"M={M}")
 
 
-# ---- the widest MFMA tiles: 64 weight rows per workgroup (NT = 4) ----
-# The host picks the most weight rows per workgroup (64, 32, 16) that still gives >= 512
-# workgroups: n_layers * ceil(R / 64) * (m-tiles / MT) >= 512 selects 64.
+# ---- qgemm_kernel's widest tiles: 64 weight rows per workgroup (NT = 4) ----
+# Where qgemm_kernel runs (up to 48 rows, or a call the LDS tiles below do not take) the host
+# picks the most weight rows per workgroup (64, 32, 16) that still gives >= 512 workgroups:
+# n_layers * ceil(R / 64) * (m-tiles / MT) >= 512 selects 64.
 
 @pytest.mark.parametrize("M", [40, 64])
 def test_qlinear_mfma_in_proj_two_layers_64_row_tiles(O, gdn, dev, M):
-    """The whole in_proj (R = 16480 rows, K = 5120) of two layers: 2 x 258 tiles of 64 rows =
-    516 workgroups, so the 64-row form runs, with 3 (M = 40) and 4 (M = 64) m-tiles."""
+    """The whole in_proj (R = 16480 rows, K = 5120) of two layers: at M = 40 2 x 258 tiles of 64
+    rows = 516 workgroups, so the 64-row form runs, with 3 m-tiles; M = 64 takes 256 of the LDS
+    tiles, with in_proj_a and in_proj_b as leftover rows."""
     import torch
     log_case(f"qlinear (MFMA path, 64-row tiles) in_proj 4 segments x 2 layers, M={M}, K=5120")
     L, K = 2, 5120
@@ -248,7 +250,7 @@ def test_qlinear_mfma_eight_layers_whole_layers_per_xcd(O, gdn, dev, M, nseg):
 
 
 # ---- 256 weight rows per workgroup, the operand shared by its four waves through LDS ----
-# One m group (M <= 64) and n_layers * ceil(R / 256) >= 512 select qgemm_ns_kernel: e.g.
+# One m group of up to 48 rows and n_layers * ceil(R / 256) >= 512 select qgemm_ns_kernel: e.g.
 # 8 layers of in_proj (65 workgroups a layer) or 26 of out_proj (20 a layer).
 
 def sampled_rows(N, rng, n=768):
@@ -262,7 +264,7 @@ def sampled_rows(N, rng, n=768):
 def test_qlinear_mfma_in_proj_rows_shared_operand(O, gdn, dev, M, K):
     """8 layers of the in_proj row count (16,480 rows in its four matrices: segment bounds
     inside workgroups, the last workgroup partly past the rows), 520 workgroups of 256 rows,
-    M from one to four m tiles; K = 1024 (8 steps of two groups, both scale and bias
+    M from one to three m tiles (M = 64 takes the LDS tiles); K = 1024 (8 steps of two groups, both scale and bias
     buffers, the repeated loads of the last steps) and K = 5120 (40 steps). At K = 5120 a
     sample of rows of every layer and segment is checked."""
     import torch
@@ -313,8 +315,8 @@ def test_qlinear_mfma_out_proj_rows_shared_operand(O, gdn, dev):
 
 
 def test_qlinear_mfma_512_rows(O, gdn, dev):
-    """The most rows the quantized path takes (512 = 32 m-tiles in 8 groups of 4), N = 4096:
-    64 tiles of 64 rows x 8 = 512 workgroups, so the 64-row form with 4 m-tiles runs."""
+    """512 rows (where the reference turns to its dequantize path), N = 4096: 32 x 8 = 256 of the
+    64 x 128 LDS tiles."""
     import torch
     log_case("qlinear (MFMA path, 64-row tiles) M=512, N=4096, K=1024")
     M, N, K = 512, 4096, 1024
@@ -330,7 +332,8 @@ def test_qlinear_mfma_512_rows(O, gdn, dev):
 
 def test_qlinear_in_proj_prefill_window_1024_rows(O, gdn, dev):
     """A 1024-token window through the layer's four in_proj matrices (K = 5120; N reduced to
-    1024 / 512 / 48 / 48 to keep the fp64 check short): 16 m groups of 64 rows, XCD-ordered."""
+    1024 / 512 / 48 / 48 to keep the fp64 check short): 12 x 16 LDS tiles of 64 operand rows,
+    XCD-ordered, and the 96 leftover rows of in_proj_a and in_proj_b."""
     import torch
     log_case("qlinear (MFMA path) in_proj 4 segments, M=1024, K=5120")
     M, K = 1024, 5120
@@ -421,6 +424,8 @@ def test_qlinear_4096_rows_two_layers(O, gdn, dev):
     (1, 260, 8192, [4096 + 7]),        # the longest K, seven leftover rows
     (1, 1000, 1024, [8000, 200, 24]),  # 128 x 256: 31 tiles + 64 rows, a partial tile, leftovers only
     (1, 897, 5120, [7936 + 255]),      # 128 x 256: a partial tile of 255 rows; one row in the last 128
+    (2, 890, 1024, [3840 + 33]),       # 128 x 256: two layers, 15 tiles (panels of 8 and 7), 210 workgroups
+    (1, 1000, 8192, [8000]),           # 128 x 256: the longest K
 ])
 def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
     import torch
@@ -441,6 +446,80 @@ def test_qlinear_lds_tiles(O, gdn, dev, L, M, K, ns):
         for l in range(L):
             check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], s[l][rows], b[l][rows]),
                   bound(O, x[l], s[l][rows], b[l][rows]), f"segment {i} layer {l}")
+
+
+def test_qlinear_lds_tiles_gated_rmsnorm(O, gdn, dev):
+    """out_proj(GatedRMSNorm(o, z)) of 1536 rows, the fewest that make it 128 x 256 tiles (20 x 12),
+    K = 6144, N = 5120; a sample of the weight rows is checked."""
+    import torch
+    log_case("qlinear (LDS tiles 128 x 256) out_proj with GatedRMSNorm, M=1536, K=6144, N=5120")
+    M, K, N = 1536, 6144, 5120
+    rng = np.random.default_rng(1801)
+    o = (rng.standard_normal((M, K)) * 0.3).astype(np.float32)
+    z = O.to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    gamma = rng.uniform(0.5, 1.5, 128).astype(np.float32)
+    _, w, s, b = quant_inputs(O, 1, M, N, K, seed=1802)
+    (y,) = gdn.qlinear([dev_mat(gdn, dev, w[0], s[0], b[0])],
+                       norm=(to_dev(o, dev), to_dev(z, dev), to_dev(gamma, dev), 1e-6))
+    torch.cuda.synchronize()
+    xn = O.gated_rmsnorm(o.reshape(-1, 128), z.reshape(-1, 128), gamma, 1e-6).reshape(M, K)
+    rows = sampled_rows(N, rng)
+    ss, bs = s[0][rows], b[0][rows]
+    wmax = (np.abs(bf16_to_f32(ss)) * 15 + np.abs(bf16_to_f32(bs))).max(axis=1)
+    flip = 3 * 2.0 ** -8 * np.abs(bf16_to_f32(xn)).max(axis=1, keepdims=True) * wmax[None, :]
+    check(to_np(y)[:, rows], O.qlinear_blocked(xn, w[0][rows], ss, bs), bound(O, xn, ss, bs) + flip, "y")
+
+
+# ---- qgemm_kernel above 48 rows: scales or biases that are 8-byte but not 16-byte aligned, and
+# matrices of fewer than 5/8 of a tile's rows ----
+
+@pytest.mark.parametrize("L,M,N,K", [
+    (1, 333, 5600, 1024),   # 64 weight rows a workgroup, 6 m groups, XCD order
+    (2, 64, 16400, 1024),   # 64 weight rows, one m group, two layers
+    (1, 333, 2800, 2048),   # 32 weight rows, XCD order
+    (1, 70, 200, 1024),     # 16 weight rows, two m groups
+    (1, 40, 300, 1024),     # up to 48 rows
+    (1, 3, 300, 1024),      # the GEMV
+])
+@pytest.mark.parametrize("which", ["scales", "biases"])
+def test_qlinear_8_byte_aligned_scales(O, gdn, dev, L, M, N, K, which):
+    import torch
+    log_case(f"qlinear (8-byte aligned {which}) L={L} M={M} N={N} K={K}")
+    rng = np.random.default_rng(M + N)
+    x, w, s, b = quant_inputs(O, L, M, N, K, seed=1900 + M + N)
+    sq = (lambda a: a) if L > 1 else (lambda a: a[0])
+    mat = dev_mat(gdn, dev, sq(w), sq(s), sq(b))
+    t = getattr(mat, which)
+    buf = torch.zeros(t.numel() + 4, dtype=t.dtype, device=dev)
+    buf[4:] = t.flatten()
+    setattr(mat, which, buf[4:].view(t.shape))
+    assert getattr(mat, which).data_ptr() % 16 == 8
+    (y,) = gdn.qlinear([mat], to_dev(sq(x), dev), n_layers=L)
+    torch.cuda.synchronize()
+    got = to_np(y).reshape(L, M, N)
+    rows = sampled_rows(N, rng) if N > 1024 else np.arange(N)
+    for l in range(L):
+        check(got[l][:, rows], O.qlinear_blocked(x[l], w[l][rows], s[l][rows], b[l][rows]),
+              bound(O, x[l], s[l][rows], b[l][rows]), f"layer {l}")
+
+
+def test_qlinear_small_matrices_4096_rows(O, gdn, dev):
+    """Four matrices of 79 rows (no 128-row tile is 5/8 full), 4096 rows, two layers."""
+    import torch
+    log_case("qlinear (qgemm, 64-row tiles) M=4096, 2 layers, 4 x 79 rows, K=1024")
+    L, M, K = 2, 4096, 1024
+    mats, host, x = [], [], None
+    for i in range(4):
+        xi, w, s, b = quant_inputs(O, L, M, 79, K, seed=2000 + i)
+        x = xi if x is None else x
+        mats.append(dev_mat(gdn, dev, w, s, b))
+        host.append((w, s, b))
+    ys = gdn.qlinear(mats, to_dev(x, dev), n_layers=L)
+    torch.cuda.synchronize()
+    for i, ((w, s, b), y) in enumerate(zip(host, ys)):
+        got = to_np(y)
+        for l in range(L):
+            check(got[l], O.qlinear_blocked(x[l], w[l], s[l], b[l]), bound(O, x[l], s[l], b[l]), f"segment {i} layer {l}")
 
 
 # ---- qgemm_kernel's 64 x 32 tiles where they are exactly two workgroups a CU (512): big_form ----
