@@ -1066,12 +1066,15 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p, QPara
 
   // The bias term sum_g (b_g - 16 s_g) sum x_g, 16 groups at a time: y += on MFMA, A = the sums x
   // of 32 operand rows x 16 groups, each split into three bf16 terms (exact to about 2^-24 of
-  // it), B = the rows' biases and their scales times -16 (exact in bf16). The large tiles (all
-  // of K in one sum) add a block's term just before its groups' products, which cancel most of
-  // it, so that y stays near its final size: with the whole term first, the share of in_proj
-  // outputs off the exact product's rounding was 1.0e-3 instead of 0.5e-3 (qgemm_kernel:
-  // 1.2e-3). With K split, the wave set wk adds every WK-th block first, while the ring fills:
-  // 4 us less at M = 333 (out_proj: 2.4e-3 to 3.1e-3 off, qgemm_kernel 2.9e-3 to 3.6e-3).
+  // it), B = the rows' biases and their scales times -16 (exact in bf16). A block's term is added
+  // just before its groups' products, which cancel most of it, so that y stays near its final
+  // size. With K split, the wave set wk adds every WK-th block, before the products of WK blocks'
+  // groups (the first while the ring fills). Shares of the outputs off the exact product's
+  // rounding at operands N(0, 1), then N(0.1, 1): large tiles (in_proj M = 1024) 0.5e-3, 1.2e-3;
+  // small tiles (M = 333) 0.8e-3, 1.4e-3; qgemm_kernel 1.2e-3, 1.5e-3. With the whole term first,
+  // as the small tiles had it, 1.0e-3 and 3.0e-3, for 1 us less of 99 (out_proj M = 333: 2.7e-3,
+  // whole term first 2.8e-3, qgemm_kernel 3.3e-3). Past a mean of about 0.2 qgemm_kernel's sums,
+  // which cancel group by group, lie nearer: N(1, 1) 4.0e-3 against 6.3e-3 and 6.4e-3.
   const int rows = 16 * p.mtiles, nks = G / 16;
   const float* const xs0 = p.xsum + (size_t)layer * G * rows;
   struct BiasBlock {
@@ -1098,9 +1101,9 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p, QPara
 #pragma unroll
     for (int i = 0; i < 8; ++i) q.v[mt][i] = xs0[off + (uint32_t)(i * rows)];
   };
-  // (inside the loop the sums are loaded here, an operand block at a time: no registers for all
-  // of them beside the loop's)
-  auto add_bias = [&](BiasBlock& q, int ks, int l) {
+  // (with `sums`, inside the loop, the sums are loaded here, an operand block at a time: no
+  // registers for all of them beside the loop's)
+  auto add_bias = [&](BiasBlock& q, int ks, int l, bool sums) {
     bf8 b0[NTW], s0[NTW];
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) {
@@ -1116,7 +1119,7 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p, QPara
     }
 #pragma unroll
     for (int mt = 0; mt < MTW; ++mt) {
-      if (WK == 1) load_sums(ks, l, mt, q);
+      if (sums) load_sums(ks, l, mt, q);
       bf8 x3[3];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -1134,22 +1137,15 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p, QPara
           y[mt][nt] = mfma32(x3[t], b0[nt], y[mt][nt]);
           y[mt][nt] = mfma32(x3[t], s0[nt], y[mt][nt]);
         }
-      if (WK == 1 && mt % 2) __builtin_amdgcn_sched_barrier(0);
+      if (sums && mt % 2) __builtin_amdgcn_sched_barrier(0);
     }
   };
   if (WK > 1 && wk < nks) {
     BiasBlock q;
-    auto load = [&](int ks) {
-      load_rows(ks, lane, q);
+    load_rows(wk, lane, q);
 #pragma unroll
-      for (int mt = 0; mt < MTW; ++mt) load_sums(ks, lane, mt, q);
-    };
-    load(wk);
-    for (int ks = wk; ks < nks; ks += WK) {
-      BiasBlock c = q;
-      load(min(ks + WK, nks - 1));
-      add_bias(c, ks, lane);
-    }
+    for (int mt = 0; mt < MTW; ++mt) load_sums(wk, lane, mt, q);
+    add_bias(q, wk, lane, false);
   }
 
   // The loop. A step's 2 MTW tiles in sequence, each tile's FMAs between the next one's MFMAs
@@ -1190,15 +1186,16 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_big_kernel(QParams p, QPara
 #pragma unroll
   for (int s = 0; s < 4; ++s) b[0][s] = nibbles16_bf16(wd[0][s], nk);
   int sl = 0;
-  constexpr int kSpan = WK == 1 ? 16 : 8;  // steps (nsteps is a multiple of it) between bias blocks, if any
-  for (int j0 = 0; j0 < nsteps; j0 += kSpan) {
-  if (WK == 1) {
+  for (int j0 = 0; j0 < nsteps; j0 += 16) {  // the steps of WK bias blocks
+  const int ks = j0 / 16 * WK + wk;
+  if (WK == 1 || (j0 > 0 && ks < nks)) {
     BiasBlock q;
     const int l = opaque_lane();
-    load_rows(j0 / kSpan, l, q);
-    add_bias(q, j0 / kSpan, l);
+    load_rows(ks, l, q);
+    add_bias(q, ks, l, true);
   }
-  for (int j = j0; j < j0 + kSpan; ++j) {
+  const int j1 = WK == 1 ? j0 + 16 : min(j0 + 16, nsteps);
+  for (int j = j0; j < j1; ++j) {
     const unsigned char* slot = ring + sl * C::kSlot;
     const int sn = sl == kBigSlots - 1 ? 0 : sl + 1;
     const unsigned char* next = ring + sn * C::kSlot;

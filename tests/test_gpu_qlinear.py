@@ -470,6 +470,35 @@ def test_qlinear_lds_tiles_gated_rmsnorm(O, gdn, dev):
     check(to_np(y)[:, rows], O.qlinear_blocked(xn, w[0][rows], ss, bs), bound(O, xn, ss, bs) + flip, "y")
 
 
+def test_qlinear_lds_tiles_keep_the_sums_near_their_size(O, gdn, dev):
+    """An operand with a small common mean, weights of zero mean (biases near -7.5 scales): the
+    offset's and the biases' terms are many times the result and cancel. The share of outputs off
+    the exact product's rounding, against qgemm_kernel's on the same values (8-byte aligned scales
+    select it), which cancels them group by group: 255,744 outputs, about 400 off in each, so a
+    quarter more is over three deviations of the difference. (With the whole bias term before the
+    products it was twice as many.)"""
+    import torch
+    log_case("qlinear (LDS tiles) operand N(0.1, 1), M=333, K=5120, N=6144")
+    M, N, K = 333, 6144, 5120
+    rng = np.random.default_rng(2100)
+    x = O.to_bf16((0.1 + rng.standard_normal((M, K))).astype(np.float32))
+    w = rng.integers(0, 2 ** 32, (N, K // 8), dtype=np.uint64).astype(np.uint32)
+    s32 = ((0.5 + rng.random((N, K // 64))) / (4.6 * K ** 0.5)).astype(np.float32)
+    s, b = O.to_bf16(s32), O.to_bf16((-s32 * (7 + rng.random((N, K // 64)))).astype(np.float32))
+    mat = dev_mat(gdn, dev, w, s, b)
+    buf = torch.zeros(mat.scales.numel() + 4, dtype=torch.bfloat16, device=dev)
+    buf[4:] = mat.scales.flatten()
+    xd = to_dev(x, dev)
+    (y,) = gdn.qlinear([mat], xd)
+    (z,) = gdn.qlinear([gdn.QuantLinear(mat.w, buf[4:].view(mat.scales.shape), mat.biases)], xd)
+    torch.cuda.synchronize()
+    rows = sampled_rows(N, rng)
+    want = O.to_bf16(O.qlinear_blocked(x, w[rows], s[rows], b[rows]).astype(np.float32))
+    off = [float((to_np(t)[:, rows] != want).mean()) for t in (y, z)]
+    print(f"  off the exact rounding: LDS tiles {off[0]:.2e}, qgemm_kernel {off[1]:.2e}", flush=True)
+    assert off[0] <= 1.25 * off[1]
+
+
 # ---- qgemm_kernel above 48 rows: scales or biases that are 8-byte but not 16-byte aligned, and
 # matrices of fewer than 5/8 of a tile's rows ----
 
