@@ -25,7 +25,7 @@
 // nibble words and the operand fragments come from the workspace; per group
 // acc = sum x (128 + q) (fp32, MFMA), then y += s * acc + (b - 128 s) * sum x. In qgemm a
 // workgroup's 4 waves split K and add their partial sums in LDS at the end, so each wave
-// reads a quarter of the operand; calls of many weight rows and one m group (up to 64 rows,
+// reads a quarter of the operand; calls of many weight rows and one m group (up to 48 rows,
 // e.g. 8 layers of in_proj at once) take qgemm_ns instead, whose workgroup of 256 weight rows
 // reads the operand into LDS once for its four waves; calls of more than 48 rows and enough
 // tiles take qgemm_big, whose workgroups share 128 x 256 or 64 x 128 tiles through LDS.
@@ -937,7 +937,7 @@ __global__ __launch_bounds__(kThreads) void qgemm_ns_kernel(QParams p) {
 // four bits: one shift more per word than 128 + q): the terms of the offset are summed apart
 // from the products that cancel them, so their size is what the fp32 sums round at, and with
 // 128 the outputs lay further from the exact product than qgemm_kernel's, which cancels them
-// group by group (with 16 they lie as near or nearer).
+// group by group (with 16 they lie as near or nearer, see the bias term in the kernel).
 typedef float f16v __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ f16v mfma32(bf8 a, bf8 b, f16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
