@@ -294,7 +294,7 @@ def _stream(stream) -> Optional[int]:
     if stream is not None:
         return stream.cuda_stream
     import torch
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # no Stream object made: 1 us less a call
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # 0.5 us a call, current_stream() 2.8
     return torch.cuda.current_stream().cuda_stream if raw is None else raw(torch.cuda.current_device())
 
 
